@@ -30,22 +30,43 @@ namespace {
 
 // invert A[layer] for the listed layers (the eliminated ones of a level, or
 // the top layer of each column) into Dinv[layer] (transposed storage)
-template <int NB>
-__global__ void __launch_bounds__(blk_nt(NB), blk_nt(NB) > NT ? 1 : 2) k_bcr_invert(int ni, int n, const int4 *__restrict__ el,
-                                                       const int2 *__restrict__ top, const int *__restrict__ off,
-                                                       const double *__restrict__ A, double *__restrict__ Dinv,
-                                                       int *__restrict__ info, const vk_colstate *__restrict__ st) {
+template <int NB, int SEARCH, int MINW>
+__global__ void __launch_bounds__(blk_nt(NB), blk_nt(NB) > NT ? 1 : MINW) k_bcr_invert(
+    int ni, int n, const int4 *__restrict__ el, const int2 *__restrict__ top, const int *__restrict__ off,
+    const double *__restrict__ A, double *__restrict__ Dinv, int *__restrict__ info,
+    const vk_colstate *__restrict__ st) {
     const int q = blockIdx.x;
     if (q >= n) return;
     const int layer = el ? el[q].x : top[q].x, c = el ? el[q].w : top[q].y;
     if (st && st[c].done) return;
+    const size_t nn = (size_t)ni * ni;
+    if (SEARCH == BLK_SEARCH_ONLY && !blk_marked(Dinv + layer * nn)) return;
     __shared__ BlkShared<NB> sh;
     if (threadIdx.x == 0) sh.info = 0;
-    const size_t nn = (size_t)ni * ni;
-    f64x4 acc[BlkGrid<NB>::TBR][BlkGrid<NB>::TBC];
-    blk_load_schur<NB>(acc, ni, A + layer * nn, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
-    blk_invert<NB>(acc, ni, Dinv + layer * nn, sh, layer - off[c] + 1);
-    if (threadIdx.x == 0 && info && sh.info) atomicCAS(&info[c], 0, sh.info);
+    blk_invert_schur<NB, SEARCH>(ni, A + layer * nn, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                 Dinv + layer * nn, sh, layer - off[c] + 1);
+    if (SEARCH != BLK_SEARCH_MARK && threadIdx.x == 0 && info && sh.info) atomicCAS(&info[c], 0, sh.info);
+}
+
+// the inversions of one launch's blocks.  Launches of at most one block per
+// CU bound a level's latency: one kernel does both inversions, with the
+// registers of one workgroup per CU.  Larger ones run diagonal pivots alone
+// at the occupancy their registers allow, then a launch that takes only the
+// blocks which refused them.
+template <int NB>
+void launch_bcr_invert(int ni, int n, const int4 *el, const int2 *top, const int *off, const double *A, double *Dinv,
+                       int *info, const vk_colstate *st, int ncu, hipStream_t s) {
+    if constexpr (blk_nt(NB) == NT) {
+        if (n <= ncu) {
+            hipLaunchKernelGGL((k_bcr_invert<NB, BLK_SEARCH_HERE, 1>), dim3(n), dim3(blk_nt(NB)), 0, s, ni, n, el, top,
+                               off, A, Dinv, info, st);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_bcr_invert<NB, BLK_SEARCH_MARK, 2>), dim3(n), dim3(blk_nt(NB)), 0, s, ni, n, el, top, off, A,
+                       Dinv, info, st);
+    hipLaunchKernelGGL((k_bcr_invert<NB, BLK_SEARCH_ONLY, 2>), dim3(n), dim3(blk_nt(NB)), 0, s, ni, n, el, top, off, A,
+                       Dinv, info, st);
 }
 
 // level 0: couplings are the diagonals Lsub (B) and Usup (C); elementwise.
@@ -517,8 +538,8 @@ int launch_bcr_factor_n(int ni, const vk_columns *cols, const double *D, const d
         const int s0 = b.surv_off[lev], ns = b.surv_off[lev + 1] - s0;
         // level 0 inverts its eliminated blocks from D (the level-0 update writes A)
         if (ne > 0)
-            hipLaunchKernelGGL((k_bcr_invert<NB>), dim3(ne), dim3(blk_nt(NB)), 0, s, ni, ne, b.d_elim + e0,
-                               (const int2 *)nullptr, cols->d_off, lev == 0 ? D : ws->A, Dinv, info, st);
+            launch_bcr_invert<NB>(ni, ne, b.d_elim + e0, nullptr, cols->d_off, lev == 0 ? D : ws->A, Dinv, info, st,
+                                  device_cus(), s);
         if (ns > 0) {
             if (lev == 0)
                 hipLaunchKernelGGL(k_bcr_update0, dim3(ns + ne, std::min(tpr * tpr, 16)), dim3(NT), 0, s, ni, ns,
@@ -532,8 +553,7 @@ int launch_bcr_factor_n(int ni, const vk_columns *cols, const double *D, const d
                                                              b.d_elim + e0, Dinv, ws, st, s);
         }
     }
-    hipLaunchKernelGGL((k_bcr_invert<NB>), dim3(b.ntop), dim3(blk_nt(NB)), 0, s, ni, b.ntop, (const int4 *)nullptr, b.d_top,
-                       cols->d_off, ws->A, Dinv, info, st);
+    launch_bcr_invert<NB>(ni, b.ntop, nullptr, b.d_top, cols->d_off, b.nlev ? ws->A : D, Dinv, info, st, device_cus(), s);
     VK_CHECK(hipGetLastError());
     return 0;
 }

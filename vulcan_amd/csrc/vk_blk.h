@@ -52,14 +52,25 @@ struct BlkShared {
     // above 128 rows the panel wave parks its accumulator tiles here during
     // the panel (its registers then hold the panel alone)
     static constexpr bool PARK = NB >= 9;
-    double pan[2][16][N16 + 1];   // panel columns, [k][row], double-buffered by panel parity
-    double rb[16][N16];           // old pivot rows of the panel, [s][col]
-    double dump[blk_nt(NB)];      // per-thread target of discarded writes
-    double prow[16];              // current pivot row of the panel factorisation
-    int ipos[N16];
-    int perm[N16];
     int info;
-    double park[PARK ? 4 * ((NB + 1) / 2) * ((NB + 3) / 4) : 1][64];
+    int refused;                      // a diagonal pivot was refused (blk_invert_diag)
+    union {
+        struct {                      // blk_invert
+            double pan[2][16][N16 + 1];   // panel columns, [k][row], double-buffered by panel parity
+            double rb[16][N16];           // old pivot rows of the panel, [s][col]
+            double dump[blk_nt(NB)];      // per-thread target of discarded writes
+            double prow[16];              // current pivot row of the panel factorisation
+            int ipos[N16];
+            int perm[N16];
+            double park[PARK ? 4 * ((NB + 1) / 2) * ((NB + 3) / 4) : 1][64];
+        };
+        struct {                      // blk_invert_diag
+            double dpan[16][N16 + 1];     // panel columns, [k][row]
+            double dfac[16][N16 + 1];     // the factored panel
+            double drb[2][16][N16];       // old pivot rows, [s][col], by panel parity
+            double diag[N16];             // the block's diagonal as given
+        };
+    };
 };
 
 template <int CTRL>
@@ -307,6 +318,183 @@ __device__ __forceinline__ void blk_invert(f64x4 (&acc)[BlkGrid<NB>::TBR][BlkGri
     __syncthreads();
 }
 
+// ---------------------------------------------------------------------------
+// The same inversion with the diagonal as pivots, for blocks that allow it.
+//
+// Searching the pivots makes the panel a serial chain on one wave: a
+// wave-wide maximum, a row hand-over through LDS and the whole panel's
+// update per step, some 900 cycles (36 of an inversion's 58 us at 93 rows)
+// while the workgroup's other waves wait.  With the pivot rows known in
+// advance, every wave holds the panel's 16 pivot rows in its lanes 0..15
+// (all waves run the same steps on them) and its own share of the other rows
+// in the lanes above, one row a lane: the pivot row of a step is lane kk's,
+// read by v_readlane into scalar registers, no row crosses waves, and a
+// panel takes two barriers instead of three (the old pivot rows are
+// published with the panel).
+//
+// Which blocks allow it: the Ros2 lhs blocks c0 I - J - diffusion and their
+// Schur complements behave like M-matrices, whose elimination in natural
+// order takes from each diagonal entry and never adds to it.  A block is
+// accepted when every pivot d has the sign of its entry a of the given block
+// and at most twice its size (a / d >= DIAG_KEEP; zero and NaN pivots fail).
+// The test does not depend on the scaling of rows or columns.  On the blocks
+// of the 30-, 93- and 150-species columns over 140 to 200 steps (dt 1e-14 to
+// 2e5 s) a / d was never below 1; the inverses were as near the exact ones
+// as with searched pivots or nearer (18 to 40 times on blocks with species
+// scaled over four decades); of 2 200 random normal matrices of 4 to 30 rows
+// 17 were accepted, all of 4 rows.  Refused blocks are inverted by
+// blk_invert (a third of the blocks in the first step from a random
+// composition).
+//
+// One column of 150 layers and 93 species: factorisation and two solves 0.77
+// -> 0.54 ms; chains of one column 5.25 -> 3.08 ms, of 256 columns (80 to 200
+// layers) 9.3 -> 6.5 ms; nine 150-species columns 17.9 -> 12.5 ms.
+// Returns whether the inverse has been written (uniform over the workgroup).
+// ---------------------------------------------------------------------------
+constexpr double DIAG_KEEP = 0.5;
+
+__device__ __forceinline__ double lane_bcast(double v, int lane) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, lane);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), lane);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+template <int NB>
+__device__ __forceinline__ bool blk_invert_diag(f64x4 (&acc)[BlkGrid<NB>::TBR][BlkGrid<NB>::TBC], int ni,
+                                                double *__restrict__ X, BlkShared<NB> &sh) {
+    using G = BlkGrid<NB>;
+    constexpr int N16 = 16 * NB, TBR = G::TBR, TBC = G::TBC, WC = G::WC;
+    constexpr int SHARE = (N16 - 16 + G::NW - 1) / G::NW;   // rows outside the pivot tile, per wave
+    static_assert(SHARE <= 48, "a wave's lanes hold the pivot rows and its share");
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));   // as in blk_load_schur: no index of this function lives across the caller's loop
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;   // uniform: the tile tests are scalar branches
+    const int wr = w / WC, wc = w % WC;
+    const int lg = l >> 4, lc = l & 15;
+    const int npan = (ni + 15) >> 4;
+    // the padding is the identity's: its pivots are 1 and touch nothing, so
+    // that every panel runs its 16 steps without a test
+#pragma unroll
+    for (int ti = 0; ti < TBR; ti++)
+#pragma unroll
+        for (int tj = 0; tj < TBC; tj++) {
+            const int bi = wr + 2 * ti, bj = wc + WC * tj;
+            if (bi != bj || bi >= NB) continue;
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (4 * r + lg == lc) {
+                    if (16 * bi + lc >= ni) acc[ti][tj][r] = 1.0;
+                    sh.diag[16 * bi + lc] = acc[ti][tj][r];
+                }
+        }
+    if (tid == 0) sh.refused = 0;
+    for (int pb = 0; pb < npan; pb++) {
+        double(*rb)[N16] = sh.drb[pb & 1];
+        const int p0 = 16 * pb;
+        // the owners of column block and row block pb publish them and clear
+        // their tiles: the update below then writes them like any other (the
+        // panel's tiles as the factored panel times the identity)
+#pragma unroll
+        for (int ti = 0; ti < TBR; ti++) {
+            const int bi = wr + 2 * ti;
+            if (bi >= NB) continue;
+#pragma unroll
+            for (int tj = 0; tj < TBC; tj++) {
+                const int bj = wc + WC * tj;
+                if (bj >= NB) continue;
+                if (bj == pb) {
+#pragma unroll
+                    for (int r = 0; r < 4; r++) sh.dpan[lc][16 * bi + 4 * r + lg] = acc[ti][tj][r];
+                    acc[ti][tj] = f64x4{0.0, 0.0, 0.0, 0.0};
+                } else if (bi == pb) {
+#pragma unroll
+                    for (int r = 0; r < 4; r++) rb[4 * r + lg][16 * bj + lc] = acc[ti][tj][r];
+                    acc[ti][tj] = f64x4{0.0, 0.0, 0.0, 0.0};
+                }
+            }
+        }
+        __syncthreads();
+        {
+            // lane -> row: the pivot rows, then this wave's share of the others
+            const int o = w * SHARE + l - 16;
+            const bool other = l >= 16 && l < 16 + SHARE && o < N16 - 16;
+            const int row = l < 16 ? p0 + l : (other ? (o < p0 ? o : o + 16) : p0);
+            double v[16], pinv = 1.0;
+#pragma unroll
+            for (int k = 0; k < 16; k++) v[k] = sh.dpan[k][row];
+#pragma unroll
+            for (int kk = 0; kk < 16; kk++) {
+                const bool own = l == kk;
+                // the pivot row, every entry into scalar registers of its own
+                // (a shared pair would serialise read and use)
+                double p[16];
+#pragma unroll
+                for (int k = 0; k < 16; k++) p[k] = lane_bcast(v[k], kk);
+                const double inv = blk_recip(p[kk]);
+                const double f = own ? 0.0 : v[kk] * inv;
+#pragma unroll
+                for (int k = 0; k < 16; k++) asm volatile("" : "+s"(p[k]));
+#pragma unroll
+                for (int j = 1; j < 16; j++) {
+                    const int k = (kk + j) & 15;      // the next pivot's column first
+                    v[k] = fma(-f, p[k], v[k]);
+                }
+                v[kk] = own ? 1.0 : -f;
+                pinv = own ? inv : pinv;
+            }
+            if (w == 0 && l < 16 && !(sh.diag[row] * pinv >= DIAG_KEEP)) sh.refused = 1;
+            if (other || (l < 16 && w == 0)) {
+#pragma unroll
+                for (int k = 0; k < 16; k++) sh.dfac[k][row] = v[k] * pinv;
+            }
+        }
+        __syncthreads();
+        if (__builtin_amdgcn_readfirstlane(sh.refused)) return false;
+        // rank-16 update on MFMA (tiles past the block read block 0's
+        // operands, their values are never used)
+        double b[TBC][4];
+#pragma unroll
+        for (int tj = 0; tj < TBC; tj++) {
+            const int bj = wc + WC * tj;
+#pragma unroll
+            for (int s4 = 0; s4 < 4; s4++) {
+                const double x = rb[4 * s4 + lg][16 * (bj < NB ? bj : 0) + lc];
+                b[tj][s4] = bj != pb ? x : (4 * s4 + lg == lc ? 1.0 : 0.0);
+            }
+        }
+#pragma unroll
+        for (int ti = 0; ti < TBR; ti++) {
+            const int bi = wr + 2 * ti;
+            double a[4];
+#pragma unroll
+            for (int s4 = 0; s4 < 4; s4++) a[s4] = sh.dfac[4 * s4 + lg][16 * (bi < NB ? bi : 0) + lc];
+#pragma unroll
+            for (int s4 = 0; s4 < 4; s4++)
+#pragma unroll
+                for (int tj = 0; tj < TBC; tj++)
+                    acc[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s4], b[tj][s4], acc[ti][tj], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int ti = 0; ti < TBR; ti++) {
+        const int bi = wr + 2 * ti;
+        if (bi >= NB) continue;
+#pragma unroll
+        for (int tj = 0; tj < TBC; tj++) {
+            const int bj = wc + WC * tj, cc = 16 * bj + lc;
+            if (bj >= NB || cc >= ni) continue;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int i = 16 * bi + 4 * r + lg;
+                if (i < ni) X[(size_t)cc * ni + i] = acc[ti][tj][r];
+            }
+        }
+    }
+    __syncthreads();
+    return true;
+}
+
 // acc = D_l - diag(cl) Xn^T diag(cn) [- diag(cl2) Xn2^T diag(cn2)] in the tile layout
 //
 // Branch-free: every thread loads all its entries unconditionally (padding
@@ -396,6 +584,49 @@ __device__ __forceinline__ void blk_load_schur(f64x4 (&acc)[BlkGrid<NB>::TBR][Bl
     };
     if (Xn) sub(cl, Xn, cn);
     if (Xn2) sub(cl2, Xn2, cn2);
+}
+
+// the workgroup's LDS for the inversions
+template <int NB>
+__device__ __forceinline__ BlkShared<NB> &blk_shared() {
+    __shared__ BlkShared<NB> sh;
+    return sh;
+}
+
+// How a kernel inverts the blocks that refuse diagonal pivots:
+enum BlkSearch {
+    BLK_SEARCH_HERE,    // in place, with searched pivots (both inversions in the kernel's registers)
+    BLK_SEARCH_MARK,    // not: their output is marked for a later launch, which takes ...
+    BLK_SEARCH_ONLY     // ... the marked blocks alone, with searched pivots
+};
+
+// The mark: a signalling NaN pattern no operation returns, in the first
+// entry of the block's output.
+constexpr unsigned long long BLK_MARK = 0x7ff4756c63616e00ull;
+
+__device__ __forceinline__ bool blk_marked(const double *X) {
+    return *(const volatile unsigned long long *)X == BLK_MARK;
+}
+
+// X = the transposed inverse of D_l - diag(cl) Xn^T diag(cn) [- diag(cl2)
+// Xn2^T diag(cn2)]; false (uniform) where X is left marked
+template <int NB, int SEARCH>
+__device__ __forceinline__ bool blk_invert_schur(int ni, const double *__restrict__ Dl, const double *cl,
+                                                 const double *Xn, const double *cn, const double *cl2,
+                                                 const double *Xn2, const double *cn2, double *__restrict__ X,
+                                                 BlkShared<NB> &sh, int tag) {
+    f64x4 acc[BlkGrid<NB>::TBR][BlkGrid<NB>::TBC];
+    if constexpr (SEARCH != BLK_SEARCH_ONLY) {
+        blk_load_schur<NB>(acc, ni, Dl, cl, Xn, cn, cl2, Xn2, cn2);
+        if (blk_invert_diag<NB>(acc, ni, X, sh)) return true;
+        if constexpr (SEARCH == BLK_SEARCH_MARK) {
+            if (threadIdx.x == 0) *(volatile unsigned long long *)X = BLK_MARK;
+            return false;
+        }
+    }
+    blk_load_schur<NB>(acc, ni, Dl, cl, Xn, cn, cl2, Xn2, cn2);
+    blk_invert<NB>(acc, ni, X, sh, tag);
+    return true;
 }
 
 // Products for the cyclic-reduction updates, one 32-row output slab (and

@@ -10,7 +10,15 @@ namespace {
 
 // 8-wave workgroups (blocks above 112 rows) run one per CU
 // (order: the chain each workgroup runs, 2c + side; null = blockIdx.x)
-template <int NB, int MINW>
+//
+// SEARCH: a chain runs with diagonal pivots (BLK_SEARCH_MARK) up to the first
+// block that refuses them, which it marks; a second launch
+// (BLK_SEARCH_ONLY) runs the rest of such chains with searched pivots.  Both
+// inversions in one kernel do not fit the registers above 128 rows (100 to
+// 290 spilled registers in the chain's loop; 13.3 -> 18.3 ms for nine
+// 150-species columns), and the second launch costs the chains that have
+// nothing left a few microseconds.
+template <int NB, int SEARCH, int MINW>
 __global__ void __launch_bounds__(blk_nt(NB), blk_nt(NB) > NT ? 1 : MINW) k_factor_blk(int ni, const int *__restrict__ off,
                                                     const int *__restrict__ order, const double *__restrict__ D,
                                                     const double *__restrict__ Lsub, const double *__restrict__ Usup,
@@ -20,53 +28,69 @@ __global__ void __launch_bounds__(blk_nt(NB), blk_nt(NB) > NT ? 1 : MINW) k_fact
     const int c = chain >> 1, side = chain & 1;
     if (st && st[c].done) return;
     __shared__ BlkShared<NB> sh;
-    if (threadIdx.x == 0) sh.info = 0;
     const int l0 = off[c], nz = off[c + 1] - l0, m = nz / 2;
     const size_t nn = (size_t)ni * ni;
-    f64x4 acc[BlkGrid<NB>::TBR][BlkGrid<NB>::TBC];
     // one loop for both chains (a single copy of the inversion code, which
     // is large: the kernel's instruction footprint matters with two
     // workgroups per CU): side 0 runs j = 0 .. m-1 coupled through Lsub_j /
     // Usup_{j-1}, side 1 runs j = nz-1 .. m+1 through Usup_j / Lsub_{j+1}
     const int dir = side == 0 ? 1 : -1, j0 = side == 0 ? 0 : nz - 1, cnt = side == 0 ? m : nz - 1 - m;
     const double *cown = side == 0 ? Lsub : Usup, *cprev = side == 0 ? Usup : Lsub;
-    for (int t = 0; t < cnt; ++t) {
+    int t = 0;
+    if constexpr (SEARCH == BLK_SEARCH_ONLY) {
+        // the first marked block: those before it hold this factorisation's
+        // inverses, those behind it whatever was there
+        if (threadIdx.x == 0) sh.refused = cnt;
+        __syncthreads();
+        for (int u = threadIdx.x; u < cnt; u += BlkGrid<NB>::NTH)
+            if (blk_marked(Dinv + (size_t)(l0 + j0 + dir * u) * nn)) atomicMin(&sh.refused, u);
+        __syncthreads();
+        t = sh.refused;
+        if (t >= cnt) return;
+    }
+    if (threadIdx.x == 0) sh.info = 0;
+    for (; t < cnt; ++t) {
         const int j = j0 + dir * t;
         const size_t l = (size_t)l0 + j, lp = (size_t)((long)l - dir);
-        blk_load_schur<NB>(acc, ni, D + l * nn, cown + l * ni, t > 0 ? Dinv + lp * nn : nullptr,
-                           t > 0 ? cprev + lp * ni : nullptr, nullptr, nullptr, nullptr);
-        blk_invert<NB>(acc, ni, Dinv + l * nn, sh, j + 1);
+        if (!blk_invert_schur<NB, SEARCH>(ni, D + l * nn, cown + l * ni, t > 0 ? Dinv + lp * nn : nullptr,
+                                          t > 0 ? cprev + lp * ni : nullptr, nullptr, nullptr, nullptr, Dinv + l * nn,
+                                          sh, j + 1))
+            return;
     }
-    if (threadIdx.x == 0 && info && sh.info) atomicCAS(&info[c], 0, sh.info);
+    if (SEARCH != BLK_SEARCH_MARK && threadIdx.x == 0 && info && sh.info) atomicCAS(&info[c], 0, sh.info);
 }
 
-template <int NB, int MINW>
+template <int NB, int SEARCH, int MINW>
 __global__ void __launch_bounds__(blk_nt(NB), blk_nt(NB) > NT ? 1 : MINW) k_factor_blk_mid(int ni, const int *__restrict__ off,
                                                         const double *__restrict__ D, const double *__restrict__ Lsub,
                                                         const double *__restrict__ Usup, double *__restrict__ Dinv,
                                                         int *__restrict__ info, const vk_colstate *__restrict__ st) {
     const int c = blockIdx.x;
     if (st && st[c].done) return;
-    __shared__ BlkShared<NB> sh;
-    if (threadIdx.x == 0) sh.info = 0;
     const int l0 = off[c], nz = off[c + 1] - l0, m = nz / 2;
     const size_t nn = (size_t)ni * ni;
     const size_t l = (size_t)l0 + m;
-    f64x4 acc[BlkGrid<NB>::TBR][BlkGrid<NB>::TBC];
-    blk_load_schur<NB>(acc, ni, D + l * nn, Lsub + l * ni, m > 0 ? Dinv + (l - 1) * nn : nullptr,
-                       m > 0 ? Usup + (l - 1) * ni : nullptr, Usup + l * ni,
-                       m < nz - 1 ? Dinv + (l + 1) * nn : nullptr, m < nz - 1 ? Lsub + (l + 1) * ni : nullptr);
-    blk_invert<NB>(acc, ni, Dinv + l * nn, sh, m + 1);
-    if (threadIdx.x == 0 && info && sh.info) atomicCAS(&info[c], 0, sh.info);
+    if (SEARCH == BLK_SEARCH_ONLY && !blk_marked(Dinv + l * nn)) return;
+    __shared__ BlkShared<NB> sh;
+    if (threadIdx.x == 0) sh.info = 0;
+    blk_invert_schur<NB, SEARCH>(ni, D + l * nn, Lsub + l * ni, m > 0 ? Dinv + (l - 1) * nn : nullptr,
+                                 m > 0 ? Usup + (l - 1) * ni : nullptr, Usup + l * ni,
+                                 m < nz - 1 ? Dinv + (l + 1) * nn : nullptr, m < nz - 1 ? Lsub + (l + 1) * ni : nullptr,
+                                 Dinv + l * nn, sh, m + 1);
+    if (SEARCH != BLK_SEARCH_MARK && threadIdx.x == 0 && info && sh.info) atomicCAS(&info[c], 0, sh.info);
 }
 
 template <int N, int MINW>
 void launch_blk(int ni, int ncols, const int *off, const int *order, const double *D, const double *Lsub,
                 const double *Usup, double *Dinv, int *info, const vk_colstate *st, hipStream_t s) {
-    hipLaunchKernelGGL((k_factor_blk<N, MINW>), dim3(2 * ncols), dim3(blk_nt(N)), 0, s, ni, off, order, D, Lsub, Usup,
-                       Dinv, info, st);
-    hipLaunchKernelGGL((k_factor_blk_mid<N, MINW>), dim3(ncols), dim3(blk_nt(N)), 0, s, ni, off, D, Lsub, Usup, Dinv, info,
-                       st);
+    hipLaunchKernelGGL((k_factor_blk<N, BLK_SEARCH_MARK, MINW>), dim3(2 * ncols), dim3(blk_nt(N)), 0, s, ni, off, order,
+                       D, Lsub, Usup, Dinv, info, st);
+    hipLaunchKernelGGL((k_factor_blk<N, BLK_SEARCH_ONLY, MINW>), dim3(2 * ncols), dim3(blk_nt(N)), 0, s, ni, off, order,
+                       D, Lsub, Usup, Dinv, info, st);
+    hipLaunchKernelGGL((k_factor_blk_mid<N, BLK_SEARCH_MARK, MINW>), dim3(ncols), dim3(blk_nt(N)), 0, s, ni, off, D,
+                       Lsub, Usup, Dinv, info, st);
+    hipLaunchKernelGGL((k_factor_blk_mid<N, BLK_SEARCH_ONLY, MINW>), dim3(ncols), dim3(blk_nt(N)), 0, s, ni, off, D,
+                       Lsub, Usup, Dinv, info, st);
 }
 
 template <int MINW>
