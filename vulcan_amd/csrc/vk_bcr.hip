@@ -1,6 +1,5 @@
 // Block cyclic reduction factorisation and solves (factor variant 4).
 #include <algorithm>
-#include <atomic>
 
 #include "vk_blk.h"
 
@@ -509,20 +508,6 @@ void launch_bcr_products(int ni, int ns, int ne, int ny, const int4 *sv, const i
                        ws->A, ws->B, ws->C, ws->P, ws->Q, st);
 }
 
-// compute units of the current device, queried once per device; 0 if the
-// query fails
-int device_cus() {
-    static std::atomic<int> cus[64];   // zero-initialised (static storage)
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-    int n = cus[dev].load(std::memory_order_relaxed);
-    if (n <= 0) {
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 0;
-        cus[dev].store(n, std::memory_order_relaxed);
-    }
-    return n;
-}
-
 template <int NB>
 int launch_bcr_factor_n(int ni, const vk_columns *cols, const double *D, const double *Lsub, const double *Usup,
                         double *Dinv, int *info, const vk_colstate *st, const vk_bcr_ws *ws, hipStream_t s) {
@@ -530,7 +515,7 @@ int launch_bcr_factor_n(int ni, const vk_columns *cols, const double *D, const d
     // deep chunks where every workgroup of a launch is resident at once,
     // at most two per CU (with three, measured slower than shallow chunks)
     constexpr long per_cu = sizeof(SlabShared<BCR_NBH<NB>, SlabKC<NB>::deep>) <= 80 * 1024 ? 2 : 1;
-    const long cap = per_cu * device_cus();
+    const long cap = per_cu * vk_device_cus();
     const int ny = (ni + 31) / 32;
     const int tpr = (ni + 31) / 32;
     for (int lev = 0; lev < b.nlev; lev++) {
@@ -539,7 +524,7 @@ int launch_bcr_factor_n(int ni, const vk_columns *cols, const double *D, const d
         // level 0 inverts its eliminated blocks from D (the level-0 update writes A)
         if (ne > 0)
             launch_bcr_invert<NB>(ni, ne, b.d_elim + e0, nullptr, cols->d_off, lev == 0 ? D : ws->A, Dinv, info, st,
-                                  device_cus(), s);
+                                  vk_device_cus(), s);
         if (ns > 0) {
             if (lev == 0)
                 hipLaunchKernelGGL(k_bcr_update0, dim3(ns + ne, std::min(tpr * tpr, 16)), dim3(NT), 0, s, ni, ns,
@@ -553,7 +538,7 @@ int launch_bcr_factor_n(int ni, const vk_columns *cols, const double *D, const d
                                                              b.d_elim + e0, Dinv, ws, st, s);
         }
     }
-    launch_bcr_invert<NB>(ni, b.ntop, nullptr, b.d_top, cols->d_off, b.nlev ? ws->A : D, Dinv, info, st, device_cus(), s);
+    launch_bcr_invert<NB>(ni, b.ntop, nullptr, b.d_top, cols->d_off, b.nlev ? ws->A : D, Dinv, info, st, vk_device_cus(), s);
     VK_CHECK(hipGetLastError());
     return 0;
 }

@@ -1,6 +1,7 @@
 // Internal structures shared by the vulcan_amd HIP sources.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <vector>
 #include "../../include/vulcan_amd.h"
 
@@ -14,6 +15,19 @@
         if (e_ != hipSuccess) return -(int)e_;                           \
     } while (0)
 
+// compute units of the current device, queried once per device; 0 if the
+// query fails
+inline int vk_device_cus() {
+    static std::atomic<int> cus[64];   // zero-initialised (static storage)
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+    int n = cus[dev].load(std::memory_order_relaxed);
+    if (n <= 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 0;
+        cus[dev].store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
 
 // one term of a Jacobian entry: coef * dv[slot] (one 16-byte load)
 // one Jacobian term packed in 32 bits: dv slot << 8 | net stoichiometric

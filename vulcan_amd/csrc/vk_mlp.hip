@@ -3,9 +3,9 @@
 //
 // GEMM: C[M][N] (fp32) = A(m,k) * B(k,n) (+ bias[n]) with A, B BF16 at
 // arbitrary (row, column) strides, so that X*W, dZ*W^T and X^T*dZ share one
-// kernel.  A 64 x 64 C tile per 256-thread workgroup, each wave one 32 x 32
-// sub-tile on v_mfma_f32_32x32x8_bf16 (k = 8 per instruction), K staged
-// through LDS in steps of 32 with both operands stored k-contiguous.
+// interface.  Operands with a unit stride go to k_gemm_tiled, others to
+// k_gemm_any.  Both run v_mfma_f32_32x32x8_bf16 over k in the same order,
+// so an output's bits do not depend on which one, or which tile, formed it.
 // Optional fused epilogue: Y = SiLU(C) written as BF16 for the next layer.
 #include "vk_internal.h"
 
@@ -25,12 +25,34 @@ __device__ __forceinline__ float bf2f(unsigned short h) { return __uint_as_float
 
 __device__ __forceinline__ float silu(float z) { return z / (1.0f + expf(-z)); }
 
+// Epilogue of a wave's 32 x 32 tile at (m0, n0): acc[q] is row 8*(q/4) +
+// 4*(lane/32) + q%4, column lane%32
+__device__ __forceinline__ void store_tile(const f32x16 &acc, int M, int N, int m0, int n0, int lane,
+                                           float *__restrict__ C, long ldc, const float *__restrict__ bias,
+                                           int accumulate, unsigned short *__restrict__ Yact, long ldy) {
+    const int col = n0 + (lane & 31);
+    if (col >= N) return;
+    const float bc = bias ? bias[col] : 0.0f;
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        const int row = m0 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
+        if (row < M) {
+            float v = acc[q];
+            if (bias) v += bc;
+            float *cp = C + (long)row * ldc + col;
+            if (accumulate) v += *cp;
+            *cp = v;
+            if (Yact) Yact[(long)row * ldy + col] = f2bf(silu(v));
+        }
+    }
+}
+
 constexpr int TM = 64, TN = 64, TK = 32, KP = TK + 4;   // LDS row pitch (in bf16) avoids bank conflicts
 
-__global__ void __launch_bounds__(256) k_gemm(int M, int N, int K, const unsigned short *__restrict__ A, long sam,
-                                              long sak, const unsigned short *__restrict__ B, long sbk, long sbn,
-                                              float *__restrict__ C, long ldc, const float *__restrict__ bias,
-                                              int accumulate, unsigned short *__restrict__ Yact, long ldy) {
+__global__ void __launch_bounds__(256) k_gemm_any(int M, int N, int K, const unsigned short *__restrict__ A, long sam,
+                                                  long sak, const unsigned short *__restrict__ B, long sbk, long sbn,
+                                                  float *__restrict__ C, long ldc, const float *__restrict__ bias,
+                                                  int accumulate, unsigned short *__restrict__ Yact, long ldy) {
     __shared__ unsigned short As[TM][KP];
     __shared__ unsigned short Bs[TN][KP];
     const int tid = threadIdx.x;
@@ -68,19 +90,238 @@ __global__ void __launch_bounds__(256) k_gemm(int M, int N, int K, const unsigne
         }
         __syncthreads();
     }
-    // acc[q]: row = 8*(q/4) + 4*(lane/32) + q%4, column = lane%32 of the wave's 32 x 32 tile
-    const int col = n0 + wn + (lane & 31);
-    for (int q = 0; q < 16; q++) {
-        const int row = m0 + wm + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
-        if (row < M && col < N) {
-            float v = acc[q];
-            if (bias) v += bias[col];
-            float *cp = C + (long)row * ldc + col;
-            if (accumulate) v += *cp;
-            *cp = v;
-            if (Yact) Yact[(long)row * ldy + col] = f2bf(silu(v));
+    store_tile(acc, M, N, m0 + wm, n0 + wn, lane, C, ldc, bias, accumulate, Yact, ldy);
+}
+
+// ---------------------------------------------------------------------------
+// The same product with both operands' unit-stride dimension read in 8- and
+// 16-byte loads.  A workgroup forms a BM x BN tile of C, each computing wave
+// WM x WN of it; all four waves stage.  K runs in chunks of KC through two
+// LDS buffers, one barrier a chunk, with the next two chunks' loads in
+// registers.  LDS holds both operands row by row
+// (row: m or n) with the 4-entry pieces of every 16 k in the order 0 2 1 3
+// (Stage::at), so that one 16-byte read gives a lane its operands of two
+// MFMAs.  An operand whose rows are the unit stride is transposed 4 x 4 in
+// registers on the way.
+//
+// An output's sum over k is one serial chain of MFMAs (32 cycles per 8 k), so
+// the tile decides how many CUs a product fills: 32 x 32 tiles, one
+// computing wave, when 64 x 64 ones would leave CUs without work, and
+// 128 x 64 ones, fewer LDS reads per MFMA, when there are two for each CU.
+//
+// Measured against k_gemm_any (two-byte loads, 64 x 64 tiles) at 256 rows:
+// 1024 x 1024 layers 123 -> 11 us (64 of the 256 CUs worked), the 1024 x
+// 13 950 head 198 -> 38 us, its weight gradient 157 -> 49 us, a training step
+// of the 307 -> 4 x 1024 -> 13 950 network 3.60 -> 0.47 ms.  The head's input
+// gradient (k = 13 950 on 32 x 32 tiles, 1 744 dependent MFMAs, 70 us) is
+// bound by that chain.
+// ---------------------------------------------------------------------------
+struct GemmArgs {
+    int M, N, K;
+    const unsigned short *A, *B;
+    long lda, ldb;               // stride of the dimension that is not the unit one
+    float *C;
+    long ldc;
+    const float *bias;
+    int accumulate;
+    unsigned short *Yact;
+    long ldy;
+};
+
+// staging registers and steps of one operand: R rows x KC; KFAST: k is the unit stride
+template <int R, int KC, bool KFAST>
+struct Stage {
+    static constexpr int PITCH = KC + 8;            // in entries: rows 16 bytes past a multiple of 128
+    static constexpr int UNITS = KFAST ? R * KC / 8 : R * KC / 16, PER = (UNITS + 255) / 256;
+    uint2 v[PER][KFAST ? 2 : 4];
+
+    // four or eight entries of a unit: whole vectors inside the operand; a
+    // tile or chunk at its edge (a uniform test) reads entry by entry with
+    // the indices clamped and zeroes what lies past it, without branches
+    __device__ __forceinline__ void load(const unsigned short *__restrict__ X, long ld, int rows, int K, int r0, int k0) {
+        const bool inside = r0 + R <= rows && k0 + KC <= K;
+        if (inside) {
+#pragma unroll
+            for (int q = 0; q < PER; q++) {
+                const int u = unit(q);
+                if constexpr (KFAST) {
+                    uint4 w;
+                    __builtin_memcpy(&w, X + (long)(r0 + u / (KC / 8)) * ld + k0 + 8 * (u % (KC / 8)), 16);
+                    v[q][0] = make_uint2(w.x, w.y);
+                    v[q][1] = make_uint2(w.z, w.w);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        __builtin_memcpy(&v[q][i], X + (long)(k0 + 4 * (u / (R / 4)) + i) * ld + r0 + 4 * (u % (R / 4)), 8);
+                }
+            }
+            return;
+        }
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            const int u = unit(q);
+            if constexpr (KFAST) {
+                const int r = r0 + u / (KC / 8), k = k0 + 8 * (u % (KC / 8));
+                const unsigned short *p = X + (long)min(r, rows - 1) * ld;
+                unsigned short e[8];
+#pragma unroll
+                for (int i = 0; i < 8; i++) e[i] = p[min(k + i, K - 1)];
+#pragma unroll
+                for (int i = 0; i < 8; i++) e[i] = r < rows && k + i < K ? e[i] : (unsigned short)0;
+                __builtin_memcpy(&v[q][0], e, 8);
+                __builtin_memcpy(&v[q][1], e + 4, 8);
+            } else {
+                const int r = r0 + 4 * (u % (R / 4)), k = k0 + 4 * (u / (R / 4));
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const unsigned short *p = X + (long)min(k + i, K - 1) * ld;
+                    unsigned short e[4];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) e[j] = p[min(r + j, rows - 1)];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) e[j] = k + i < K && r + j < rows ? e[j] : (unsigned short)0;
+                    __builtin_memcpy(&v[q][i], e, 8);
+                }
+            }
         }
     }
+
+    // threads past the last unit stage one that another thread stages too
+    static __device__ __forceinline__ int unit(int q) {
+        const int u = threadIdx.x + 256 * q;
+        return UNITS % 256 != 0 ? u % UNITS : u;
+    }
+
+    // entry of the 4-entry piece c (k = 4 c ..) of a row: 16-byte granules of
+    // two pieces, a granule's place exchanged within four by bits 4 and 5 of
+    // the row (the transposing stores write rows 4 apart, whose banks repeat
+    // every 16 rows without it: 8 conflict cycles an access; the reads of 16
+    // consecutive rows stay free of conflicts)
+    static __device__ __forceinline__ int at(int r, int c) {
+        return r * PITCH + 8 * (((c >> 2) * 2 + (c & 1)) ^ ((r >> 4) & 3)) + 4 * ((c >> 1) & 1);
+    }
+
+    __device__ __forceinline__ void store(unsigned short *sm) const {
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            const int u = unit(q);
+            if constexpr (KFAST) {
+                const int r = u / (KC / 8), c = 2 * (u % (KC / 8));
+                *(uint2 *)(sm + at(r, c)) = v[q][0];
+                *(uint2 *)(sm + at(r, c + 1)) = v[q][1];
+            } else {
+                const int r = 4 * (u % (R / 4)), c = u / (R / 4);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    // entry j of the four k rows
+                    const unsigned sel = j & 1 ? 0x07060302u : 0x05040100u;
+                    const unsigned x0 = j < 2 ? v[q][0].x : v[q][0].y, x1 = j < 2 ? v[q][1].x : v[q][1].y;
+                    const unsigned x2 = j < 2 ? v[q][2].x : v[q][2].y, x3 = j < 2 ? v[q][3].x : v[q][3].y;
+                    *(uint2 *)(sm + at(r + j, c)) =
+                        make_uint2(__builtin_amdgcn_perm(x1, x0, sel), __builtin_amdgcn_perm(x3, x2, sel));
+                }
+            }
+        }
+    }
+};
+
+template <int BM, int BN, int WM, int WN, int KC, bool AK, bool BK>
+__global__ void __launch_bounds__(256, BM == 128 ? 2 : 4) k_gemm_tiled(GemmArgs g) {
+    using SA = Stage<BM, KC, AK>;
+    using SB = Stage<BN, KC, BK>;
+    constexpr int P = SA::PITCH, TA = WM / 32, TB = WN / 32, WX = BN / WN, NWC = (BM / WM) * WX;
+    static_assert(NWC <= 4, "four waves");
+    __shared__ __align__(16) unsigned short sm[2][(BM + BN) * P];
+    // workgroups go to the 8 XCDs in turn: each XCD takes a contiguous range
+    // of tiles, m fastest, so that the tiles sharing B's columns share an L2
+    const int tm = (g.M + BM - 1) / BM, tiles = tm * ((g.N + BN - 1) / BN), per = (tiles + 7) / 8;
+    const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+    if ((int)(blockIdx.x / 8) >= per || t >= tiles) return;
+    const int m0 = BM * (t % tm), n0 = BN * (t / tm);
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wm = WM * (w / WX), wn = WN * (w % WX);
+    const bool computes = NWC == 4 || w < NWC;
+    f32x16 acc[TA][TB];
+#pragma unroll
+    for (int i = 0; i < TA; i++)
+#pragma unroll
+        for (int j = 0; j < TB; j++)
+#pragma unroll
+            for (int q = 0; q < 16; q++) acc[i][j][q] = 0.0f;
+    // a lane's operands of two MFMAs (16 k from k) of the 32 rows from r0
+    auto operand = [&](int r0, int k) {
+        const int r = r0 + (lane & 31);
+        return r * P + 8 * ((k / 8 + (lane >> 5)) ^ ((r >> 4) & 3));
+    };
+    // chunk c + 1 waits in registers while chunk c is multiplied, c + 2 is in
+    // flight
+    constexpr int AHEAD = 2;
+    SA sa[AHEAD];
+    SB sb[AHEAD];
+    const int nch = (g.K + KC - 1) / KC;
+    auto load = [&](int slot, int c) {
+        if (c < nch) {
+            sa[slot].load(g.A, g.lda, g.M, g.K, m0, c * KC);
+            sb[slot].load(g.B, g.ldb, g.N, g.K, n0, c * KC);
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < AHEAD; d++) load(d, d);
+    sa[0].store(sm[0]);
+    sb[0].store(sm[0] + BM * P);
+    load(0, AHEAD);
+    for (int c0 = 0; c0 < nch; c0 += AHEAD) {
+#pragma unroll
+        for (int d = 0; d < AHEAD; d++) {
+            const int c = c0 + d, slot = (d + 1) % AHEAD;
+            if (c >= nch) break;
+            // the other buffer's readers (chunk c - 1) are past this barrier
+            __syncthreads();
+            if (computes) {
+                const unsigned short *pa = sm[c & 1], *pb = pa + BM * P;
+#pragma unroll
+                for (int k = 0; k < KC; k += 16) {
+                    bf16x4 a[TA][2], b[TB][2];
+#pragma unroll
+                    for (int i = 0; i < TA; i++)
+                        __builtin_memcpy(a[i], __builtin_assume_aligned(pa + operand(wm + 32 * i, k), 16), 16);
+#pragma unroll
+                    for (int j = 0; j < TB; j++)
+                        __builtin_memcpy(b[j], __builtin_assume_aligned(pb + operand(wn + 32 * j, k), 16), 16);
+#pragma unroll
+                    for (int h = 0; h < 2; h++)
+#pragma unroll
+                        for (int i = 0; i < TA; i++)
+#pragma unroll
+                            for (int j = 0; j < TB; j++)
+                                acc[i][j] =
+                                    __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a[i][h], b[j][h], acc[i][j], 0, 0, 0);
+                }
+            }
+            if (c + 1 < nch) {
+                sa[slot].store(sm[(c + 1) & 1]);
+                sb[slot].store(sm[(c + 1) & 1] + BM * P);
+                load(slot, c + 1 + AHEAD);
+            }
+        }
+    }
+    if (computes)
+#pragma unroll
+        for (int i = 0; i < TA; i++)
+#pragma unroll
+            for (int j = 0; j < TB; j++)
+                store_tile(acc[i][j], g.M, g.N, m0 + wm + 32 * i, n0 + wn + 32 * j, lane, g.C, g.ldc, g.bias,
+                           g.accumulate, g.Yact, g.ldy);
+}
+
+template <int BM, int BN, int WM, int WN, int KC>
+void launch_gemm(const GemmArgs &g, bool ak, bool bk, hipStream_t s) {
+    const long tiles = (long)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
+    const dim3 grid((unsigned)(8 * ((tiles + 7) / 8)));
+    if (ak && bk) hipLaunchKernelGGL((k_gemm_tiled<BM, BN, WM, WN, KC, true, true>), grid, dim3(256), 0, s, g);
+    else if (ak) hipLaunchKernelGGL((k_gemm_tiled<BM, BN, WM, WN, KC, true, false>), grid, dim3(256), 0, s, g);
+    else if (bk) hipLaunchKernelGGL((k_gemm_tiled<BM, BN, WM, WN, KC, false, true>), grid, dim3(256), 0, s, g);
+    else hipLaunchKernelGGL((k_gemm_tiled<BM, BN, WM, WN, KC, false, false>), grid, dim3(256), 0, s, g);
 }
 
 // dZ = dY * silu'(Z), written as fp32 and BF16; silu'(z) = s (1 + z (1 - s)), s = sigmoid(z)
@@ -119,12 +360,24 @@ __global__ void k_mse(long n, const float *__restrict__ Y, const float *__restri
     if (threadIdx.x == 0) loss_part[blockIdx.x] = red[0];
 }
 
-// column sums: out[n] = sum_m X[m][n]  (bias gradients), fixed order
-__global__ void k_colsum(int M, int N, const float *__restrict__ X, float *__restrict__ out) {
-    int n = blockIdx.x * blockDim.x + threadIdx.x;
+// column sums: out[n] = sum_m X[m][n]  (bias gradients), in order of m.  One
+// thread per column, one wave per workgroup (a hidden layer's 1024 columns
+// on 16 CUs), 16 rows' loads in flight ahead of their sums: a load at a time
+// took a memory round trip per row (26 us for 256 x 1024).
+__global__ void __launch_bounds__(64) k_colsum(int M, int N, const float *__restrict__ X, float *__restrict__ out) {
+    const int n = blockIdx.x * 64 + threadIdx.x;
     if (n >= N) return;
+    const float *p = X + n;
     float s = 0.0f;
-    for (int m = 0; m < M; m++) s += X[(long)m * N + n];
+    int m = 0;
+    for (; m + 16 <= M; m += 16) {
+        float x[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) x[i] = p[(long)(m + i) * N];
+#pragma unroll
+        for (int i = 0; i < 16; i++) s += x[i];
+    }
+    for (; m < M; m++) s += p[(long)m * N];
     out[n] = s;
 }
 
@@ -157,10 +410,23 @@ extern "C" int vk_mlp_gemm(int M, int N, int K, const void *d_A, long sam, long 
                            long sbn, float *d_C, long ldc, const float *d_bias, int accumulate, void *d_Yact,
                            long ldy, void *stream) {
     if (M <= 0 || N <= 0 || K <= 0 || !d_A || !d_B || !d_C) return VK_EINVAL;
-    dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM);
-    hipLaunchKernelGGL(k_gemm, grid, dim3(256), 0, (hipStream_t)stream, M, N, K, (const unsigned short *)d_A, sam,
-                       sak, (const unsigned short *)d_B, sbk, sbn, d_C, ldc, d_bias, accumulate,
-                       (unsigned short *)d_Yact, ldy);
+    hipStream_t s = (hipStream_t)stream;
+    // the tiled kernel where each operand has a unit stride
+    const bool ak = sak == 1, am = sam == 1, bk = sbk == 1, bn = sbn == 1;
+    if ((ak || am) && (bk || bn)) {
+        const GemmArgs g = {M, N, K, (const unsigned short *)d_A, (const unsigned short *)d_B, ak ? sam : sak,
+                            bk ? sbn : sbk, d_C, ldc, d_bias, accumulate, (unsigned short *)d_Yact, ldy};
+        const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64), t128 = (long)((M + 127) / 128) * ((N + 63) / 64);
+        const int ncu = vk_device_cus();
+        if (t128 >= 2L * ncu) launch_gemm<128, 64, 64, 32, 64>(g, ak, bk, s);
+        else if (t64 >= ncu) launch_gemm<64, 64, 32, 32, 64>(g, ak, bk, s);
+        else launch_gemm<32, 32, 32, 32, 128>(g, ak, bk, s);
+    } else {
+        dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM);
+        hipLaunchKernelGGL(k_gemm_any, grid, dim3(256), 0, s, M, N, K, (const unsigned short *)d_A, sam, sak,
+                           (const unsigned short *)d_B, sbk, sbn, d_C, ldc, d_bias, accumulate,
+                           (unsigned short *)d_Yact, ldy);
+    }
     VK_CHECK(hipGetLastError());
     return 0;
 }
@@ -184,7 +450,7 @@ extern "C" int vk_mlp_mse(long n, const float *d_Y, const float *d_T, const floa
 
 extern "C" int vk_mlp_colsum(int M, int N, const float *d_X, float *d_out, void *stream) {
     if (M <= 0 || N <= 0 || !d_X || !d_out) return VK_EINVAL;
-    hipLaunchKernelGGL(k_colsum, grid1(N), dim3(256), 0, (hipStream_t)stream, M, N, d_X, d_out);
+    hipLaunchKernelGGL(k_colsum, dim3((N + 63) / 64), dim3(64), 0, (hipStream_t)stream, M, N, d_X, d_out);
     VK_CHECK(hipGetLastError());
     return 0;
 }
