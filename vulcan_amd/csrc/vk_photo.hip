@@ -10,7 +10,7 @@
 // flux) rows off[c] .. of [L][nbin].  One thread per (column, wavelength
 // bin) sweeps the layers: every bin is independent, and consecutive threads
 // read consecutive bins of a row (coalesced).
-#include <atomic>
+#include <algorithm>
 
 #include "vk_internal.h"
 #include "vk_device.h"
@@ -175,36 +175,337 @@ __global__ void __launch_bounds__(PT) k_photo_flux(PhotoDev ph, const int *__res
         atomicMax(&ph.change[c], (unsigned long long)__double_as_longlong(red[0]));
 }
 
-// photolysis rates of every branch (op.py:2751-2787): trapezoidal sums over
-// the two uniform bin widths; the branch's rate column of k = J f_diurnal.  One
-// workgroup per layer, one wave per branch, the layer's actinic flux in LDS.
-__global__ void __launch_bounds__(PT) k_photo_J(PhotoDev ph, const int *__restrict__ layer_col, int nr,
-                                                double *__restrict__ k) {
-    extern __shared__ double af[];
-    const int l = blockIdx.x;
-    const int c = layer_col[l];
-    if (!ph.due[c]) return;
-    const int nb = ph.nbin;
-    for (int b = threadIdx.x; b < nb; b += PT) af[b] = ph.aflux[(size_t)l * nb + b];
-    __syncthreads();
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int d = ph.din12 >= 0 ? ph.din12 : nb - 1;
-    for (int br = w; br < ph.nbranch; br += PT / 64) {
-        const int tt = ph.br_T[br];
-        const double *cr = tt >= 0 ? ph.cross_J_T + ((size_t)tt * ph.L + l) * nb : ph.cross_J + (size_t)br * nb;
-        double s1 = 0.0, s2 = 0.0;
-        for (int b = lane; b < d; b += 64) s1 += af[b] * cr[b] * ph.dbin1;
-        for (int b = d + lane; b < nb; b += 64) s2 += af[b] * cr[b] * ph.dbin2;
-        for (int m = 32; m > 0; m >>= 1) {
-            s1 += __shfl_xor(s1, m);
-            s2 += __shfl_xor(s2, m);
+// ---------------------------------------------------------------------------
+// The same optical depth and fluxes by two kernels that do what a layer
+// contributes on its own for many layers at once, and leave to one thread
+// per bin the running sum of the optical depth and the sweeps' few serial
+// operations.  Every value is formed by the operations of k_photo_tau and
+// k_photo_flux in their order.  A thread per bin doing all of it (k_photo_tau, k_photo_flux)
+// keeps 10 workgroups busy for one column, each waiting on memory and on the
+// coefficients' latency layer after layer.  150 layers of 2 588 bins: 583 us
+// each before, 15 us (k_photo_layers, bound by reading the cross sections
+// from L2) and 37 us (k_photo_rt, a third of it the serial parts) now; 48
+// columns: 1 125 us each before, 170 and 777 us now (three workgroups per CU
+// by LDS).
+// ---------------------------------------------------------------------------
+
+// every layer's own optical depth (left in the tau row of its lower level)
+// and single-scattering albedo (op.py:2580-2601, 2627-2639); PT bins and
+// TAU_LAYERS layers per workgroup, so that a cross section is read once per
+// TAU_LAYERS layers
+constexpr int TAU_LAYERS = 8, TAU_SPECIES = 32;   // species per round through LDS
+
+__global__ void __launch_bounds__(PT, 4) k_photo_layers(PhotoDev ph, int ni, const int *__restrict__ layer_col,
+                                                     const double *__restrict__ y, const double *__restrict__ ymix,
+                                                     const double *__restrict__ dz) {
+    __shared__ double ny[TAU_SPECIES][TAU_LAYERS], mx[TAU_SPECIES][TAU_LAYERS];   // y dz and ymix
+    const int l0 = TAU_LAYERS * blockIdx.y, nl = min(TAU_LAYERS, ph.L - l0), nb = ph.nbin;
+    const int b = min((int)(blockIdx.x * PT + threadIdx.x), nb - 1);
+    const bool mine = blockIdx.x * PT + threadIdx.x < nb;
+    bool any = false;
+    for (int q = 0; q < nl; q++) any = any || ph.due[layer_col[l0 + q]];
+    if (!any) return;
+    double t[TAU_LAYERS], tabs[TAU_LAYERS], tscat[TAU_LAYERS];
+#pragma unroll
+    for (int q = 0; q < TAU_LAYERS; q++) t[q] = tabs[q] = tscat[q] = 0.0;
+    // the species of a round: absorbers, then scatterers
+    auto stage = [&](const int *list, int a0, int n) {
+        __syncthreads();
+        for (int e = threadIdx.x; e < n * TAU_LAYERS; e += PT) {
+            const int a = e / TAU_LAYERS, q = e % TAU_LAYERS, l = l0 + min(q, nl - 1), sp = list[a0 + a];
+            ny[a][q] = y[(size_t)l * ni + sp] * dz[l];
+            mx[a][q] = ymix[(size_t)l * ni + sp];
         }
-        if (lane == 0) {
-            double J = s1;
-            J -= 0.5 * (af[0] * cr[0] + af[d - 1] * cr[d - 1]) * ph.dbin1;
-            J += s2;
-            J -= 0.5 * (af[d] * cr[d] + af[nb - 1] * cr[nb - 1]) * ph.dbin2;
-            k[(size_t)l * nr + ph.br_col[br]] = J * ph.f_diurnal;
+        __syncthreads();
+    };
+    for (int a0 = 0; a0 < ph.nabs; a0 += TAU_SPECIES) {
+        const int n = min(TAU_SPECIES, ph.nabs - a0);
+        stage(ph.abs_sp, a0, n);
+#pragma unroll 2
+        for (int a = 0; a < n; a++) {
+            const int tt = ph.abs_T[a0 + a];
+            const double cr = ph.cross[(size_t)(a0 + a) * nb + b];
+            if (tt >= 0) {
+                const double *ct = ph.cross_T + ((size_t)tt * ph.L + l0) * nb + b;
+                double crt[TAU_LAYERS];
+#pragma unroll
+                for (int q = 0; q < TAU_LAYERS; q++) crt[q] = ct[(size_t)min(q, nl - 1) * nb];
+#pragma unroll
+                for (int q = 0; q < TAU_LAYERS; q++) t[q] += ny[a][q] * crt[q];
+            } else {
+#pragma unroll
+                for (int q = 0; q < TAU_LAYERS; q++) t[q] += ny[a][q] * cr;
+            }
+#pragma unroll
+            for (int q = 0; q < TAU_LAYERS; q++) tabs[q] += mx[a][q] * cr;
+        }
+    }
+    for (int a0 = 0; a0 < ph.nscat; a0 += TAU_SPECIES) {
+        const int n = min(TAU_SPECIES, ph.nscat - a0);
+        stage(ph.scat_sp, a0, n);
+        for (int a = 0; a < n; a++) {
+            const double cr = ph.cross_scat[(size_t)(a0 + a) * nb + b];
+#pragma unroll
+            for (int q = 0; q < TAU_LAYERS; q++) {
+                t[q] += ny[a][q] * cr;
+                tscat[q] += mx[a][q] * cr;
+            }
+        }
+    }
+    if (!mine) return;
+#pragma unroll
+    for (int q = 0; q < TAU_LAYERS; q++) {
+        if (q >= nl) break;
+        const int l = l0 + q, c = layer_col[l];
+        if (!ph.due[c]) continue;
+        double w = tscat[q] / (tabs[q] + tscat[q]);
+        if (w != w) w = 0.0;                       // nan_to_num: 0/0
+        ph.tau[(size_t)(l + c) * nb + b] = t[q];
+        ph.w0[(size_t)l * nb + b] = fmin(w, 1. - 1.E-8);
+    }
+}
+
+// optical depth of the levels, direct beam, both sweeps, actinic flux
+// (op.py:2603-2738): RT_BINS bins of a column per workgroup, 32 threads per
+// bin.  A sweep's step is
+//     F[j] = 1/chi (phi F[j'] - xi G + i / mu)
+// with G the other flux at the layer's far level, known ahead of the
+// downward sweep from the previous update, and of the upward one from the
+// downward: xi G is formed ahead too, and four operations a layer stay
+// serial, in the reference's order (as one multiply-add with 1/chi taken
+// into the constants they lose six digits where xi G and i / mu cancel).
+// RT_ARRAYS doubles per bin and level in LDS: the serial parts' latency is
+// hidden by the other workgroups of a CU, so what a thread alone uses later
+// (xi and i / mu of its up to RT_LANES-spaced R layers) waits in its
+// registers, and the downward flux in global memory.  Columns of up to 416
+// layers run here; longer ones keep k_photo_tau and k_photo_flux.
+constexpr int RT_BINS = 8, RT_LANES = PT / RT_BINS, RT_ARRAYS = 4, RT_RUN = 8, RT_ROUNDS = 13;
+
+constexpr size_t rt_lds(int nz) { return sizeof(double) * RT_ARRAYS * RT_BINS * (size_t)(nz + 1); }
+
+// f = inv (phi f - xg + F) over n layers from j in steps of dj, f into F;
+// RT_RUN layers are read ahead of the chain and written behind it (a store
+// between two layers' loads would put an LDS round trip into every step)
+__device__ __forceinline__ void rt_sweep(const double *inv, const double *phi, const double *xg, double *F, int j, int dj,
+                                         int n, double f) {
+    for (int q0 = 0; q0 < n; q0 += RT_RUN) {
+        double i[RT_RUN], p[RT_RUN], x[RT_RUN], v[RT_RUN];
+#pragma unroll
+        for (int q = 0; q < RT_RUN; q++) {
+            const int e = RT_BINS * (j + dj * min(q0 + q, n - 1));
+            i[q] = inv[e]; p[q] = phi[e]; x[q] = xg[e]; v[q] = F[e];
+        }
+#pragma unroll
+        for (int q = 0; q < RT_RUN; q++) v[q] = f = i[q] * (p[q] * f - x[q] + v[q]);
+#pragma unroll
+        for (int q = 0; q < RT_RUN; q++)
+            if (q0 + q < n) F[RT_BINS * (j + dj * (q0 + q))] = v[q];
+    }
+}
+
+// R: rounds of RT_LANES layers that cover the longest column
+template <int R>
+__global__ void __launch_bounds__(PT) k_photo_rt(PhotoDev ph, const int *__restrict__ off) {
+    extern __shared__ double rt[];
+    const int c = blockIdx.y;
+    if (!ph.due[c]) return;
+    const int o = off[c], nz = off[c + 1] - o, nb = ph.nbin, span = RT_BINS * (nz + 1);
+    const int bl = threadIdx.x % RT_BINS, j0 = threadIdx.x / RT_BINS;
+    const bool mine = blockIdx.x * RT_BINS + bl < nb;
+    const int b = min((int)blockIdx.x * RT_BINS + bl, nb - 1);
+    // [level][bin] each; F holds i / mu until the fluxes replace it
+    double *inv = rt + bl, *phi = inv + span, *xg = phi + span, *F = xg + span;
+    const size_t base = (size_t)(o + c) * nb + b;           // level 0 of the column
+    auto at = [](int j) { return j * RT_BINS; };
+    double *tau = inv;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int j = j0 + RT_LANES * r;
+        if (j < nz) tau[at(j)] = ph.tau[base + (size_t)j * nb];
+    }
+    __syncthreads();
+    if (j0 == 0) {
+        double above = 0.0;
+        tau[at(nz)] = 0.0;
+        for (int j = nz - 1; j >= 0; j -= RT_RUN) {
+            double v[RT_RUN];
+#pragma unroll
+            for (int u = 0; u < RT_RUN; u++) v[u] = tau[at(max(j - u, 0))];
+#pragma unroll
+            for (int u = 0; u < RT_RUN; u++) v[u] = above = v[u] + above;
+#pragma unroll
+            for (int u = 0; u < RT_RUN; u++)
+                if (j - u >= 0) tau[at(j - u)] = v[u];
+        }
+    }
+    __syncthreads();
+    const double mu = -1. * ph.cos_sl, top = ph.sflux_top[b];
+    double *sf = xg;
+    for (int j = j0; j <= nz; j += RT_LANES) {
+        const double t = tau[at(j)], f = top * exp(-1. * t / ph.cos_sl);
+        sf[at(j)] = f;
+        F[at(j)] = t;                    // tau again, for the layers' differences
+        if (mine) {
+            ph.tau[base + (size_t)j * nb] = t;
+            ph.sflux[base + (size_t)j * nb] = f;
+        }
+    }
+    __syncthreads();
+    // the coefficients take tau's and the beam's places a round of layers
+    // behind their reads
+    double xi[R], iu[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int j = j0 + RT_LANES * r;
+        TwoStream t = {};
+        double prev = 0.0;
+        if (j < nz) {
+            t = two_stream(ph, mu, ph.w0[(size_t)(o + j) * nb + b], F[at(j)] - F[at(j + 1)], sf[at(j)] * ph.cos_sl,
+                           sf[at(j + 1)] * ph.cos_sl);
+            prev = ph.dflux_u[base + (size_t)j * nb];
+        }
+        __syncthreads();
+        if (j < nz) {
+            inv[at(j)] = 1. / t.chi;
+            phi[at(j)] = t.phi;
+            xg[at(j)] = t.xi * prev;
+            F[at(j)] = t.i_d / mu;
+        }
+        xi[r] = t.xi;
+        iu[r] = t.i_u / mu;
+    }
+    __syncthreads();
+    if (j0 == 0) {
+        const double d = ph.dflux_d[base + (size_t)nz * nb];
+        F[at(nz)] = d;
+        rt_sweep(inv, phi, xg, F, nz - 1, -1, nz, d);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int j = j0 + RT_LANES * r;
+        if (j < nz) {
+            xg[at(j)] = xi[r] * F[at(j + 1)];
+            if (mine) ph.dflux_d[base + (size_t)j * nb] = F[at(j)];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int j = j0 + RT_LANES * r;
+        if (j < nz) F[at(j)] = iu[r];
+    }
+    __syncthreads();
+    // the upward flux of level j + 1 in layer j's place
+    if (j0 == 0) rt_sweep(inv, phi, xg, F, 0, 1, nz, ph.dflux_u[base]);
+    __syncthreads();
+    // actinic flux and the largest relative change over the bins above flux_atol
+    double mx = 0.0;
+    if (mine) {
+        const double hc = ph.hc_bin[b];
+        for (int j = j0; j < nz; j += RT_LANES) {
+            const size_t lj = base + (size_t)j * nb;
+            const double ulo = j > 0 ? F[at(j - 1)] : ph.dflux_u[base], uhi = F[at(j)];
+            const double ave = 0.5 * (ph.sflux[lj] + ph.sflux[lj + nb]);
+            const double tot = ave + 0.5 * (ulo + uhi + ph.dflux_d[lj + nb] + ph.dflux_d[lj]) / ph.edd;
+            const double af = tot / hc;
+            ph.dflux_u[lj + nb] = uhi;
+            double *ap = ph.aflux + (size_t)(o + j) * nb + b;
+            const double prev = *ap;
+            *ap = af;
+            if (af > ph.flux_atol) {
+                const double ch = fabs(af - prev) / af;
+                if (ch == ch) mx = fmax(mx, ch);
+            }
+        }
+    }
+    for (int m = 32; m > 0; m >>= 1) mx = fmax(mx, __shfl_xor(mx, m));
+    // positive doubles order as their bit patterns
+    if ((threadIdx.x & 63) == 0 && mx > 0.0)
+        atomicMax(&ph.change[c], (unsigned long long)__double_as_longlong(mx));
+}
+
+template <int R>
+void launch_photo_rt(const PhotoDev &d, const vk_columns *cols, hipStream_t s) {
+    hipLaunchKernelGGL((k_photo_rt<R>), dim3((d.nbin + RT_BINS - 1) / RT_BINS, cols->ncols), dim3(PT),
+                       rt_lds(cols->max_nz), s, d, cols->d_off);
+}
+
+// photolysis rates of every branch (op.py:2751-2787): trapezoidal sums over
+// the two uniform bin widths; the branch's rate column of k = J f_diurnal.
+// One wave per branch for the LT layers of a workgroup, whose actinic flux
+// is in LDS.  The cross sections are read once per workgroup from L2 (36
+// branches of 2 588 bins: 0.75 MB; at one layer each, 48 columns read 4.8 GB
+// in 0.65 ms; at four 0.38 ms), so batches take as many layers as LDS holds; a column or two
+// take one, with the branches split over the grid's y dimension to fill the
+// device.
+constexpr int J_NT = 1024, J_LDS = 10400;   // doubles: four layers of 2 600 bins, or one of 8 192
+
+// STAGE: the actinic flux through LDS (spectra beyond J_LDS bins read it from
+// memory for every branch)
+template <int LT, bool STAGE = true>
+__global__ void __launch_bounds__(J_NT) k_photo_J(PhotoDev ph, const int *__restrict__ layer_col, int nr,
+                                                  double *__restrict__ k) {
+    __shared__ double lds[STAGE ? J_LDS : 1];
+    const int l0 = LT * blockIdx.x, nb = ph.nbin, nl = min(LT, ph.L - l0);
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = J_NT / 64;
+    const bool due = lane < nl && ph.due[layer_col[l0 + min(lane, nl - 1)]];   // lane: layer
+    if (!__any(due)) return;
+    const double *af = ph.aflux + (size_t)l0 * nb;
+    if constexpr (STAGE) {
+#pragma unroll 8
+        for (int e = threadIdx.x; e < LT * nb; e += J_NT) {
+            const double a = af[min(e, nl * nb - 1)];
+            lds[e] = e < nl * nb ? a : 0.0;
+        }
+        __syncthreads();
+        af = lds;
+    }
+    const int d = ph.din12 >= 0 ? ph.din12 : nb - 1;
+    for (int br = w + nw * blockIdx.y; br < ph.nbranch; br += nw * gridDim.y) {
+        const int tt = ph.br_T[br];
+        const double *cr = tt >= 0 ? ph.cross_J_T + ((size_t)tt * ph.L + l0) * nb : ph.cross_J + (size_t)br * nb;
+        // the next layer's table (the last layer's own where there is none)
+        auto row = [&](int q) { return tt >= 0 ? cr + (size_t)min(q, nl - 1) * nb : cr; };
+        double s1[LT], s2[LT];
+#pragma unroll
+        for (int q = 0; q < LT; q++) s1[q] = s2[q] = 0.0;
+        auto sum = [&](double (&s)[LT], int b0, int b1, double width) {
+            if (tt >= 0) {
+#pragma unroll 4
+                for (int b = b0 + lane; b < b1; b += 64)
+#pragma unroll
+                    for (int q = 0; q < LT; q++) s[q] += af[q * nb + b] * row(q)[b] * width;
+            } else {
+#pragma unroll 8
+                for (int b = b0 + lane; b < b1; b += 64) {
+                    const double x = cr[b];
+#pragma unroll
+                    for (int q = 0; q < LT; q++) s[q] += af[q * nb + b] * x * width;
+                }
+            }
+        };
+        sum(s1, 0, d, ph.dbin1);
+        sum(s2, d, nb, ph.dbin2);
+        // lane q finishes layer q
+        const double *x = row(lane), *a = af + min(lane, LT - 1) * nb;
+        const double x0 = x[0], x1 = x[d - 1], x2 = x[d], x3 = x[nb - 1];
+        double t1 = 0.0, t2 = 0.0;
+#pragma unroll
+        for (int q = 0; q < LT; q++) {
+            for (int m = 32; m > 0; m >>= 1) {
+                s1[q] += __shfl_xor(s1[q], m);
+                s2[q] += __shfl_xor(s2[q], m);
+            }
+            t1 = lane == q ? s1[q] : t1;
+            t2 = lane == q ? s2[q] : t2;
+        }
+        if (due) {
+            double J = t1;
+            J -= 0.5 * (a[0] * x0 + a[d - 1] * x1) * ph.dbin1;
+            J += t2;
+            J -= 0.5 * (a[d] * x2 + a[nb - 1] * x3) * ph.dbin2;
+            k[(size_t)(l0 + lane) * nr + ph.br_col[br]] = J * ph.f_diurnal;
         }
     }
 }
@@ -298,11 +599,33 @@ int vk_launch_photo(vk_photo *ph, const vk_plan *plan, const vk_columns *cols, c
     const int nc = cols->ncols;
     hipLaunchKernelGGL(k_photo_due, dim3((nc + 127) / 128), dim3(128), 0, s, nc, st, force, ini_frq, final_frq,
                        yconv_min, d.last, d.switched, d.due, d.change);
-    const dim3 grid((d.nbin + PT - 1) / PT, nc);
-    hipLaunchKernelGGL(k_photo_tau, grid, dim3(PT), 0, s, d, plan->ni, cols->d_off, y, ymix, dz);
-    hipLaunchKernelGGL(k_photo_flux, grid, dim3(PT), 0, s, d, cols->d_off);
-    const size_t smem = sizeof(double) * (size_t)d.nbin;
-    hipLaunchKernelGGL(k_photo_J, dim3(cols->L), dim3(PT), smem, s, d, cols->d_layer_col, plan->nr, k);
+    if (cols->max_nz <= RT_LANES * RT_ROUNDS) {
+        hipLaunchKernelGGL(k_photo_layers, dim3((d.nbin + PT - 1) / PT, (cols->L + TAU_LAYERS - 1) / TAU_LAYERS), dim3(PT),
+                           0, s, d, plan->ni, cols->d_layer_col, y, ymix, dz);
+        switch ((cols->max_nz + RT_LANES - 1) / RT_LANES) {
+        case 1: case 2: case 3: launch_photo_rt<3>(d, cols, s); break;
+        case 4: case 5: launch_photo_rt<5>(d, cols, s); break;
+        case 6: case 7: launch_photo_rt<7>(d, cols, s); break;
+        default: launch_photo_rt<RT_ROUNDS>(d, cols, s);
+        }
+    } else {
+        const dim3 grid((d.nbin + PT - 1) / PT, nc);
+        hipLaunchKernelGGL(k_photo_tau, grid, dim3(PT), 0, s, d, plan->ni, cols->d_off, y, ymix, dz);
+        hipLaunchKernelGGL(k_photo_flux, grid, dim3(PT), 0, s, d, cols->d_off);
+    }
+    const int L = cols->L, ncu = std::max(1, vk_device_cus());
+    if (4 * d.nbin <= J_LDS && L >= 8 * ncu)
+        hipLaunchKernelGGL(k_photo_J<4>, dim3((L + 3) / 4), dim3(J_NT), 0, s, d, cols->d_layer_col, plan->nr, k);
+    else if (2 * d.nbin <= J_LDS && L >= 4 * ncu)
+        hipLaunchKernelGGL(k_photo_J<2>, dim3((L + 1) / 2), dim3(J_NT), 0, s, d, cols->d_layer_col, plan->nr, k);
+    else {
+        // about two workgroups per CU, at least a branch per wave
+        const int gy = std::max(1, std::min((d.nbranch + J_NT / 64 - 1) / (J_NT / 64), (2 * ncu + L - 1) / L));
+        if (d.nbin <= J_LDS)
+            hipLaunchKernelGGL(k_photo_J<1>, dim3(L, gy), dim3(J_NT), 0, s, d, cols->d_layer_col, plan->nr, k);
+        else
+            hipLaunchKernelGGL((k_photo_J<1, false>), dim3(L, gy), dim3(J_NT), 0, s, d, cols->d_layer_col, plan->nr, k);
+    }
     hipLaunchKernelGGL(k_photo_change, dim3((nc + 127) / 128), dim3(128), 0, s, nc, d.due, d.change, st);
     VK_CHECK(hipGetLastError());
     return 0;
