@@ -48,6 +48,22 @@ __global__ void __launch_bounds__(blk_nt(NB), blk_nt(NB) > NT ? 1 : MINW) k_fact
         t = sh.refused;
         if (t >= cnt) return;
     }
+    if constexpr (SEARCH == BLK_SEARCH_MARK) {
+        // the inverse stays in the accumulators for the next block's Schur term
+        f64x4 acc[BlkGrid<NB>::TBR][BlkGrid<NB>::TBC];
+        for (; t < cnt; ++t) {
+            const size_t l = (size_t)l0 + j0 + dir * t;
+            if (t == 0)
+                blk_load_schur<NB>(acc, ni, D + l * nn, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+            else
+                blk_next_schur<NB>(acc, ni, D + l * nn, cown + l * ni, cprev + (size_t)((long)l - dir) * ni);
+            if (!blk_invert_diag<NB>(acc, ni, Dinv + l * nn, sh)) {
+                if (threadIdx.x == 0) *(volatile unsigned long long *)(Dinv + l * nn) = BLK_MARK;
+                return;
+            }
+        }
+        return;
+    }
     if (threadIdx.x == 0) sh.info = 0;
     for (; t < cnt; ++t) {
         const int j = j0 + dir * t;
