@@ -50,224 +50,271 @@ __global__ void k_zero_int(int n, int *__restrict__ p) {
 }
 
 // ---------------------------------------------------------------------------
-// Twisted block solves, 1024-thread workgroups.  Thread (i, h) = (tid % RP,
-// tid / RP) owns species row i and the h-th of SP column chunks of each
-// inverse (SolveShape below), so one layer's matrix-vector product is
-// SP-way split, and the Dinv chunks of the next layers (SolveDepth) are in
-// flight while the current layer is processed (the chain over layers is
-// latency bound, not bandwidth bound).
+// Twisted block solves, one workgroup per chain.  Wave w owns rows
+// [w CH, w CH + CH) of each transposed inverse and forms their share of every
+// sum; a lane holds C neighbouring columns, one 8- to 24-byte load per row.
+// After the step's one barrier G lanes add the W shares of each of the wave's
+// own species, which is all the wave needs for its rows of the next step
+// (handed out with readlane), and keep that species' couplings and
+// right-hand side.
+//
+// Everything a step reads from memory is issued DEP steps ahead.  The loads
+// stay in flight only because nothing waits for more than it needs: the loop
+// is unrolled DEP times instead of moving buffers down (a move waits for the
+// load), has no exit but its end and no access that a branch skips (the count
+// of what is in flight stays known); rows past the block and steps past the
+// end are buffer accesses out of range, which load zero and store nothing.
+// 256 columns of 80 to 200 layers, 93 species: 675 -> 512 us a sweep (3.7 ->
+// 4.8 TB/s; the kernel before moved its buffers down and so had one layer in
+// flight); 80 columns of 100 to 150 layers, 150 species: 565 -> 465 us (160
+// chains leave 96 CUs idle); one column of 60 layers, 30 species: 22 -> 18 us
+// (0.45 us a step: barrier, LDS round trip and 70 instructions of one wave).
 // Both sweeps stay within the column: layer indices run over [0, nz).
 // ---------------------------------------------------------------------------
-constexpr int NTS = 1024;
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
-// rows per part (64, 128, or the padded block size 16 NB above 128
-// species), parts (16 or 8; 7 or 6 for NB 9 or 10: threads from SP * RP on
-// hold no part) and column chunk per thread (CH <= 27 doubles, so that one
-// layer's chunk stays in registers at 1024 threads; CH <= 16 (NB - 1) + 1,
-// the fewest species of NB blocks, so a chunk always fits in the block)
-template <int NB>
-struct SolveShape {
-    static constexpr int RP = 16 * NB <= 64 ? 64 : (16 * NB <= 128 ? 128 : 16 * NB);
-    static constexpr int SP = NTS / RP;
-    static constexpr int CH = (16 * NB + SP - 1) / SP;
-    static_assert(SP * RP <= NTS && SP * CH >= 16 * NB && CH <= 16 * (NB - 1) + 1, "solve shape");
-};
-
-// Where a thread's chunk of a layer's inverse lies: rows mb .. mb+CH-1 of
-// the transposed inverse (column ib).  A part's chunk starts at m0 = h CH;
-// the last part's is moved back to end at row ni-1 (mb = ni - CH) and its
-// first d = m0 - mb entries, which belong to the part before, are zeroed;
-// rows i >= ni read column ni-1 (their sums are never used) and threads
-// without a part read part 0's chunk.  Every load stays inside the block.
-struct ChunkMap {
-    int voff;   // byte offset of (mb, ib) in the block
-    int d;      // leading entries to zero
-    int mb;     // first row of the chunk
-};
-
-template <int SP, int CH>
-__device__ __forceinline__ ChunkMap chunk_map(int ni, int i, int h) {
-    const int m0 = (h < SP ? h : 0) * CH;
-    const int mb = min(m0, ni - CH);
-    return {(mb * ni + min(i, ni - 1)) * 8, m0 - mb, mb};
+// v plus the value of the lane that the DPP control CTRL pairs this one with
+template <int CTRL>
+__device__ __forceinline__ double add_pair(double v) {
+    const u32x2 b = __builtin_bit_cast(u32x2, v);
+    const u32x2 o = {(unsigned)__builtin_amdgcn_mov_dpp((int)b[0], CTRL, 0xf, 0xf, true),
+                     (unsigned)__builtin_amdgcn_mov_dpp((int)b[1], CTRL, 0xf, 0xf, true)};
+    return v + __builtin_bit_cast(double, o);
 }
 
-// r[q] = Xt[mb + q][ib] (zero for q < d): raw buffer loads with the
-// thread's offset in one register and the uniform row stride q ni in the
-// scalar offset, over the block's byte range
-template <int CH>
-__device__ __forceinline__ void load_chunk(double (&r)[CH], const double *__restrict__ Xt, int ni,
-                                           const ChunkMap &cm) {
-    const __amdgpu_buffer_rsrc_t rs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(Xt), (short)0, ni * ni * 8, 0x00020000);
+// W CH >= 16 NB rows, 64 C >= 16 NB columns; C <= 16 (NB - 1) + 1, so a
+// lane's columns always fit in the block.  16 waves at no more than 128
+// registers keep DEP layers of one chain in flight on a CU; blocks of up to 64
+// species have too few rows for that many.  DEP steps' loads and stores stay
+// below the 63 a wave can track.
+template <int NB>
+struct Sweep {
+    static constexpr int C = NB <= 4 ? 1 : (NB <= 8 ? 2 : 3);
+    static constexpr int W = NB == 1 ? 4 : (NB <= 4 ? 8 : 16);
+    static constexpr int CH = 16 * NB / W;
+    static constexpr int G = CH <= 4 ? W : (CH <= 8 ? 8 : 4);    // lanes per species: CH G <= 64
+    static constexpr int DEP = NB <= 4 ? 4 : (NB <= 6 ? 3 : (NB <= 8 ? 2 : 1));
+    static constexpr int NTH = 64 * W, MINW = NB <= 4 ? 2 : 4;
+    static constexpr int RP = 64 * C + 8;                        // row pitch: G rows on different banks
+    static_assert(W * CH == 16 * NB && 64 * C >= 16 * NB && C <= 16 * (NB - 1) + 1 && CH * G <= 64 && W % G == 0,
+                  "sweep shape");
+    typedef double Share[W][RP];
+
+    int ni, w, cs, from, rr, own;
+    int voff[CH];
+    bool in;
+
+    __device__ __forceinline__ Sweep(int n) {
+        ni = n;
+        const int lane = threadIdx.x & 63;
+        w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+        const int c0 = min(C * lane, ni - C);               // first column of the lane
+        cs = C * lane < ni ? c0 : C * lane;                 // lanes past the block: columns that nobody reads
 #pragma unroll
-    for (int q = 0; q < CH; q++) {
-        const double x = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, cm.voff, q * ni * 8, 0));
-        r[q] = q >= cm.d ? x : 0.0;
+        for (int q = 0; q < CH; q++) voff[q] = ((w * CH + q) * ni + c0) * 8;
+        const int q = lane / G, row = w * CH + q;           // species whose sum the lane helps to add
+        in = q < CH && row < ni;
+        rr = min(row, ni - 1) * 8;
+        from = (lane % G) * RP + (rr >> 3);
+        own = in && lane % G == 0 ? rr : 0x7ffffff0;        // out of any buffer: the store is dropped
     }
-}
 
-// layers in flight per thread: fewer for larger blocks (128 registers per thread at 1024 threads)
-template <int NB>
-struct SolveDepth {
-    static constexpr int value = NB <= 4 ? 4 : (NB <= 5 ? 3 : (NB <= 8 ? 2 : 1));
+    // n doubles at p as a buffer, or nothing
+    static __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const double *p, int n, bool on) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(p), (short)0, on ? n * 8 : 0, 0x00020000);
+    }
+    // the lane's species from a layer's row of a (layer, species) array, and to it
+    __device__ __forceinline__ double get(const double *p, bool on = true) const {
+        return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(buffer(p, ni, on), rr, 0, 0));
+    }
+    __device__ __forceinline__ void put(double *p, double x, bool on = true) const {
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), buffer(p, ni, on), own, 0, 0);
+    }
+
+    // r[q][e] = Xt[w CH + q][c0 + e], zero for rows past the block
+    __device__ __forceinline__ void load(double (&r)[CH][C], const double *Xt, bool on) const {
+        const __amdgpu_buffer_rsrc_t rs = buffer(Xt, ni * ni, on);
+#pragma unroll
+        for (int q = 0; q < CH; q++) {
+            if constexpr (C >= 2) {
+                const f64x2 x = __builtin_bit_cast(f64x2, __builtin_amdgcn_raw_buffer_load_b128(rs, voff[q], 0, 0));
+                r[q][0] = x[0];
+                r[q][1] = x[1];
+            }
+            if constexpr (C != 2)
+                r[q][C - 1] =
+                    __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, voff[q] + 8 * (C - 1), 0, 0));
+        }
+    }
+
+    // the wave's share of the sums; v: the value of the lane's species
+    __device__ __forceinline__ void product(const double (&r)[CH][C], double v, Share &share) const {
+        double y[C] = {};
+        v = in ? v : 0.0;
+#pragma unroll
+        for (int q = 0; q < CH; q++) {
+            const double vq = lane_bcast(v, q * G);
+#pragma unroll
+            for (int e = 0; e < C; e++) y[e] = fma(r[q][e], vq, y[e]);
+        }
+#pragma unroll
+        for (int e = 0; e < C; e++) share[w][cs + e] = y[e];
+    }
+
+    // the lane's species from all waves' shares, in two parts: what the lane
+    // reads, and the sum over its group
+    __device__ __forceinline__ void shares(double (&y)[W / G], const Share &share) const {
+#pragma unroll
+        for (int h = 0; h < W / G; h++) y[h] = (&share[0][0])[from + h * G * RP];
+    }
+    static __device__ __forceinline__ double total(const double (&p)[W / G]) {
+        double y = p[0];
+#pragma unroll
+        for (int h = 1; h < W / G; h++) y += p[h];
+        y = add_pair<0xB1>(y);                      // quad_perm 1 0 3 2
+        y = add_pair<0x4E>(y);                      // quad_perm 2 3 0 1
+        if (G == 8) y = add_pair<0x141>(y);         // row_half_mirror
+        return y;
+    }
 };
 
-template <int DEP, int CH>
-__device__ __forceinline__ void rotate(double (&b)[DEP][CH]) {
-#pragma unroll
-    for (int d = 0; d + 1 < DEP; d++) {
-#pragma unroll
-        for (int q = 0; q < CH; q++) b[d][q] = b[d + 1][q];
-    }
-}
-
-// y_i = sum_m Xt[m][i] v[m] from the registers of the row parts; the result
-// is valid in threads h == 0 (i < ni).  One barrier (part is double-buffered
-// by the callers).
-template <int SP, int RP, int CH>
-__device__ __forceinline__ double solve_matvec(const double (&cur)[CH], const double *v, double (*part)[RP], int i,
-                                               int h, int m0) {
-    double acc = 0.0;
-#pragma unroll
-    for (int q = 0; q < CH; q++) acc = fma(cur[q], v[m0 + q], acc);
-    if (h < SP) part[h][i] = acc;
-    __syncthreads();
-    double y = part[0][i];
-#pragma unroll
-    for (int hh = 1; hh < SP; hh++) y += part[hh][i];
-    return y;
-}
-
 template <int NB>
-__global__ void __launch_bounds__(NTS) k_solve_fwd2(int ni, const int *__restrict__ off, const int *__restrict__ order,
-                                                     const double *__restrict__ Dinv, const double *__restrict__ Lsub,
-                                                     const double *__restrict__ Usup, const double *in, double *tmp,
-                                                     const vk_colstate *__restrict__ st) {
-    constexpr int RP = SolveShape<NB>::RP, SP = SolveShape<NB>::SP, CH = SolveShape<NB>::CH;
+__global__ void __launch_bounds__(Sweep<NB>::NTH, Sweep<NB>::MINW)
+    k_solve_fwd(int ni, const int *__restrict__ off, const int *__restrict__ order, const double *__restrict__ Dinv,
+                const double *__restrict__ Lsub, const double *__restrict__ Usup, const double *in, double *tmp,
+                const vk_colstate *__restrict__ st) {
+    using W = Sweep<NB>;
+    constexpr int DEP = W::DEP;
     const int chain = order ? order[blockIdx.x] : (int)blockIdx.x;   // 2c + side
     const int c = chain >> 1, side = chain & 1;
     if (st && st[c].done) return;
-    const int tid = threadIdx.x, i = tid % RP, h = tid / RP;
-    const ChunkMap cm = chunk_map<SP, CH>(ni, i, h);
+    const W sw(ni);
     const int l0 = off[c], nz = off[c + 1] - l0, m = nz / 2;
-    const size_t nn = (size_t)ni * ni;
-    // v and part double-buffered by step parity: two barriers per step; the
-    // right-hand side and coupling of the next step are loaded a step ahead
-    __shared__ double v[2][SP * CH];
-    __shared__ double part[2][SP][RP];
-    for (int q = tid; q < 2 * SP * CH; q += NTS) v[q / (SP * CH)][q % (SP * CH)] = 0.0;
+    __shared__ __align__(16) typename W::Share share[2];         // by step parity: one barrier a step
     const int j0 = side == 0 ? 0 : nz - 1, dj = side == 0 ? 1 : -1;
     const int nsteps = side == 0 ? m : nz - 1 - m;
-    const double *cpl = side == 0 ? Lsub : Usup;
-    constexpr int DEP = SolveDepth<NB>::value;
-    double buf[DEP][CH];
-#pragma unroll
-    for (int d = 0; d < DEP; d++)
-        if (d < nsteps) load_chunk<CH>(buf[d], Dinv + (size_t)(l0 + j0 + d * dj) * nn, ni, cm);
-    const bool row = h == 0 && i < ni;
-    double zi = 0.0, in_n = 0.0, cp_n = 0.0;
-    if (row && nsteps > 0) {
-        in_n = in[(size_t)(l0 + j0) * ni + i];
-        cp_n = cpl[(size_t)(l0 + j0) * ni + i];
-    }
-    __syncthreads();
-    for (int s = 0; s < nsteps; s++) {
-        const size_t l = (size_t)(l0 + j0 + dj * s);
-        const int pb = s & 1;
-        const double in_s = in_n, cp_s = cp_n;
-        if (row && s + 1 < nsteps) {
-            in_n = in[(l + dj) * ni + i];
-            cp_n = cpl[(l + dj) * ni + i];
-        }
-        if (row) {
-            double w = in_s;
-            if (s > 0) w = w - cp_s * zi;
-            v[pb][i] = w;
-        }
+    // where the next load and store lie; they end on the last layer
+    const size_t first = (size_t)(l0 + j0);
+    const double *pD = Dinv + first * ni * ni, *pi = in + first * ni, *pc = (side == 0 ? Lsub : Usup) + first * ni;
+    double *pt = tmp + first * ni;
+    double buf[DEP][W::CH][W::C], inb[DEP], cpb[DEP];
+    auto load = [&](int d, int s) {
+        const bool on = s < nsteps;
+        const long go = s + 1 < nsteps ? dj * ni : 0;
+        inb[d] = sw.get(pi, on);
+        cpb[d] = sw.get(pc, on);
+        sw.load(buf[d], pD, on);
+        pi += go;
+        pc += go;
+        pD += go * ni;
+    };
+    double y[W::W / W::G];
+    auto step = [&](int d, int s, double v) {
+        sw.product(buf[d], v, share[s & 1]);
+        __builtin_amdgcn_sched_barrier(0);        // the new loads into the registers just read
+        load(d, s + DEP);
         __syncthreads();
-        const double z = solve_matvec<SP, RP, CH>(buf[0], v[pb], part[pb], i, h, cm.mb);
-        if (row) {
-            tmp[l * ni + i] = z;
-            zi = z;
+        sw.shares(y, share[s & 1]);
+    };
+#pragma unroll
+    for (int d = 0; d < DEP; d++) load(d, d);
+    step(0, 0, inb[0]);
+    // step s closes step s - 1; those past the end (up to a multiple of DEP)
+    // load and store nothing
+    for (int s0 = 1; s0 <= nsteps; s0 += DEP) {
+#pragma unroll
+        for (int e = 0; e < DEP; e++) {
+            const int s = s0 + e, d = (1 + e) % DEP;
+            const double z = sw.total(y);
+            sw.put(pt, z, s <= nsteps);
+            pt += s < nsteps ? dj * ni : 0;
+            step(d, s, inb[d] - cpb[d] * z);
         }
-        rotate<DEP, CH>(buf);
-        if (s + DEP < nsteps) load_chunk<CH>(buf[DEP - 1], Dinv + (size_t)(l0 + j0 + dj * (s + DEP)) * nn, ni, cm);
     }
     // park b_m in the unused slot m so the backward kernel never reads `in`
     // (which may alias `out`)
-    if (side == 0 && h == 0 && i < ni) {
-        const size_t lm = (size_t)l0 + m;
-        tmp[lm * ni + i] = in[lm * ni + i];
-    }
+    if (side == 0) sw.put(tmp + ((size_t)l0 + m) * ni, sw.get(in + ((size_t)l0 + m) * ni));
 }
 
-template <int NB>
-__global__ void __launch_bounds__(NTS) k_solve_bwd2(int ni, const int *__restrict__ off, const int *__restrict__ order,
-                                                     const double *__restrict__ Dinv, const double *__restrict__ Lsub,
-                                                     const double *__restrict__ Usup, const double *tmp, double *out,
-                                                     const vk_colstate *__restrict__ st, double *acc) {
-    constexpr int RP = SolveShape<NB>::RP, SP = SolveShape<NB>::SP, CH = SolveShape<NB>::CH;
+template <int NB, bool ACC>
+__global__ void __launch_bounds__(Sweep<NB>::NTH, Sweep<NB>::MINW)
+    k_solve_bwd(int ni, const int *__restrict__ off, const int *__restrict__ order, const double *__restrict__ Dinv,
+                const double *__restrict__ Lsub, const double *__restrict__ Usup, const double *tmp, double *out,
+                const vk_colstate *__restrict__ st, double *acc) {
+    using W = Sweep<NB>;
+    constexpr int DEP = W::DEP;
     const int chain = order ? order[blockIdx.x] : (int)blockIdx.x;   // 2c + side
     const int c = chain >> 1, side = chain & 1;
     if (st && st[c].done) return;
-    const int tid = threadIdx.x, i = tid % RP, h = tid / RP;
-    const ChunkMap cm = chunk_map<SP, CH>(ni, i, h);
+    const W sw(ni);
     const int l0 = off[c], nz = off[c + 1] - l0, m = nz / 2;
-    const size_t nn = (size_t)ni * ni;
-    __shared__ double v[2][SP * CH];
-    __shared__ double part[2][SP][RP];
-    for (int q = tid; q < 2 * SP * CH; q += NTS) v[q / (SP * CH)][q % (SP * CH)] = 0.0;
-    const size_t lm = (size_t)l0 + m;
+    const size_t lm = ((size_t)l0 + m) * ni;
+    __shared__ __align__(16) typename W::Share share[2];
     const int dj = side == 0 ? -1 : 1;
     const int nsteps = 1 + (side == 0 ? m : nz - 1 - m);     // the middle layer, then the chain outwards
-    const double *cpl = side == 0 ? Usup : Lsub;
-    constexpr int DEP = SolveDepth<NB>::value;
-    double buf[DEP][CH];
-#pragma unroll
-    for (int d = 0; d < DEP; d++)
-        if (d < nsteps) load_chunk<CH>(buf[d], Dinv + (size_t)((long)lm + (long)d * dj) * nn, ni, cm);
-    const bool row = h == 0 && i < ni;
-    // x_m = M^-1 (b_m - Lsub_m z_{m-1} - Usup_m w_{m+1}); both sides compute it
-    if (row) {
-        double w = tmp[lm * ni + i];
-        if (m > 0) w = w - Lsub[lm * ni + i] * tmp[(lm - 1) * ni + i];
-        if (m < nz - 1) w = w - Usup[lm * ni + i] * tmp[(lm + 1) * ni + i];
-        v[0][i] = w;
-    }
-    // coupling and forward-sweep value of the next layer, a step ahead
-    double cp_n = 0.0, t_n = 0.0;
-    if (row && nsteps > 1) {
-        cp_n = cpl[(lm + dj) * ni + i];
-        t_n = tmp[(lm + dj) * ni + i];
-    }
-    __syncthreads();
-    double xi = solve_matvec<SP, RP, CH>(buf[0], v[0], part[0], i, h, cm.mb);
-    if (side == 0 && row) {
-        out[lm * ni + i] = xi;
-        if (acc) acc[lm * ni + i] = acc[lm * ni + i] + xi;
-    }
-    rotate<DEP, CH>(buf);
-    if (DEP < nsteps) load_chunk<CH>(buf[DEP - 1], Dinv + (size_t)((long)lm + (long)DEP * dj) * nn, ni, cm);
-    for (int s = 1; s < nsteps; s++) {
-        const size_t l = lm + (long)dj * s;
-        const int pb = s & 1;
-        const double cp_s = cp_n, t_s = t_n;
-        if (row && s + 1 < nsteps) {
-            cp_n = cpl[(l + dj) * ni + i];
-            t_n = tmp[(l + dj) * ni + i];
+    const double *pD = Dinv + lm * ni, *pc = (side == 0 ? Usup : Lsub) + lm, *pt = tmp + lm;
+    const double *pa = acc + (ACC ? lm : 0);
+    double *po = out + lm, *pao = acc + (ACC ? lm : 0);
+    double buf[DEP][W::CH][W::C], cpb[DEP], tb[DEP], ab[DEP];
+    auto load = [&](int d, int s) {
+        const bool on = s < nsteps;
+        const long go = s + 1 < nsteps ? dj * ni : 0;
+        cpb[d] = sw.get(pc, on);
+        sw.load(buf[d], pD, on);
+        pc += go;
+        pD += go * ni;
+    };
+    // what the end of step s needs, which falls into step s + 1
+    auto load_end = [&](int d, int s) {
+        const bool on = s < nsteps;
+        const long go = s + 1 < nsteps ? dj * ni : 0;
+        tb[d] = sw.get(pt, on);
+        pt += go;
+        if (ACC) {
+            ab[d] = sw.get(pa, on);
+            pa += go;
         }
-        if (row) v[pb][i] = cp_s * xi;
+    };
+    double y[W::W / W::G];
+    auto step = [&](int d, int s, double v) {
+        sw.product(buf[d], v, share[s & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        load(d, s + DEP);
         __syncthreads();
-        const double y = solve_matvec<SP, RP, CH>(buf[0], v[pb], part[pb], i, h, cm.mb);
-        if (row) {
-            xi = t_s - y;
-            out[l * ni + i] = xi;
-            if (acc) acc[l * ni + i] = acc[l * ni + i] + xi;
+        sw.shares(y, share[s & 1]);
+    };
+    // the solution of step s from its shares; the middle layer (the shares'
+    // sum itself) is stored by one side
+    auto finish = [&](int d, int s) {
+        const double z = sw.total(y), x = s == 0 ? z : tb[d] - z;
+        const bool on = s >= side && s < nsteps;
+        const long go = s + 1 < nsteps ? dj * ni : 0;
+        sw.put(po, x, on);
+        po += go;
+        if (ACC) {
+            sw.put(pao, ab[d] + x, on);
+            pao += go;
         }
-        rotate<DEP, CH>(buf);
-        if (s + DEP < nsteps)
-            load_chunk<CH>(buf[DEP - 1], Dinv + (size_t)((long)lm + (long)dj * (s + DEP)) * nn, ni, cm);
+        return x;
+    };
+#pragma unroll
+    for (int d = 0; d < DEP; d++) {
+        load(d, d);
+        load_end(d, d);
+    }
+    // x_m = M^-1 (b_m - Lsub_m z_{m-1} - Usup_m w_{m+1}); both sides compute it
+    double v = tb[0];
+    if (m > 0) v = v - sw.get(Lsub + lm) * sw.get(tmp + lm - ni);
+    if (m < nz - 1) v = v - sw.get(Usup + lm) * sw.get(tmp + lm + ni);
+    step(0, 0, v);
+    for (int s0 = 1; s0 <= nsteps; s0 += DEP) {
+#pragma unroll
+        for (int e = 0; e < DEP; e++) {
+            const double x = finish(e, s0 + e - 1);
+            load_end(e, s0 + e - 1 + DEP);
+            step((1 + e) % DEP, s0 + e, cpb[(1 + e) % DEP] * x);
+        }
     }
 }
 
@@ -395,11 +442,14 @@ template <int NB>
 void launch_solve_n(int ni, int ncols, const int *off, const int *order, const double *Dinv, const double *Lsub,
                     const double *Usup, const double *in, double *out, double *tmp, const vk_colstate *st, double *acc,
                     hipStream_t s) {
-    hipLaunchKernelGGL((k_solve_fwd2<NB>), dim3(2 * ncols), dim3(NTS), 0, s, ni, off, order, Dinv, Lsub, Usup, in, tmp,
-                       st);
-    hipLaunchKernelGGL((k_solve_bwd2<NB>), dim3(2 * ncols), dim3(NTS), 0, s, ni, off, order, Dinv, Lsub, Usup, tmp, out,
-                       st, acc);
+    const dim3 grid(2 * ncols), block(Sweep<NB>::NTH);
+    hipLaunchKernelGGL((k_solve_fwd<NB>), grid, block, 0, s, ni, off, order, Dinv, Lsub, Usup, in, tmp, st);
+    if (acc)
+        hipLaunchKernelGGL((k_solve_bwd<NB, true>), grid, block, 0, s, ni, off, order, Dinv, Lsub, Usup, tmp, out, st, acc);
+    else
+        hipLaunchKernelGGL((k_solve_bwd<NB, false>), grid, block, 0, s, ni, off, order, Dinv, Lsub, Usup, tmp, out, st, acc);
 }
+
 }  // namespace
 
 // acc (nullable): also add the solution into acc, row by row as it is written
