@@ -39,110 +39,220 @@ __device__ __forceinline__ int vk_ix(int i, int n, int site) {
 namespace {
 
 constexpr int BLK = 256;
+constexpr int RATE_LAYERS = 8;   // layers of a workgroup of k_rates, at most
 
 // ---------------------------------------------------------------------------
 // rates (op.py:145-207, 287-309; photolysis op.py:2786)
 // ---------------------------------------------------------------------------
 
-__global__ void k_grt(int L, int ni, const double *__restrict__ Tco, const double *__restrict__ nasa9,
-                      double *__restrict__ grt) {
-    int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= L * ni) return;
-    int l = idx / ni, s = idx - l * ni;
-    grt[idx] = g_RT(Tco[l], nasa9 + 20 * s);
+// One workgroup per LG layers: what depends on a layer alone (log T in two
+// doubles, powers of T, g/RT of every species) is formed once and kept in LDS,
+// and a thread keeps a pair's parameters and species for all its layers.
+// T^n exp(-E/T) and the reverse constant's exp(dG/RT) take one exponential
+// each, of an argument held in two doubles, instead of a pow, an exp and a
+// division; arguments or results near the ends of the range (and NaN) take
+// the library functions.  256 columns (36 000 layers), 93 species, 620 pairs:
+// 493 us in two kernels, with g/RT written and read back, -> 255 us (bound by
+// FP64 arithmetic; the 360 MB of rates take 75 us); the largest error against
+// 64 bits is the same 2.4e-15.
+
+struct LayerRate {
+    double T, rT, lh, ll;              // 1/T, log T = lh + ll (NaN: no fast path)
+    double M, emtau, x, rx;            // exp(-tau), CORR T and its inverse
+    double logT, T2, T3, T4;
+};
+
+// g/RT = h/RT - s/R of the NASA9 polynomials (thermo/gibbs_text.txt:13-18),
+// low set below 1000 K, high set at and above (chem_funs.py:2789-2792)
+__device__ inline double g_layer(const LayerRate &y, const double *a20) {
+    const double *a = a20 + (y.T < 1000.0 ? 0 : 10);
+    const double h = -a[0] / y.T2 + a[1] * y.logT / y.T + a[2] + a[3] * y.T / 2. + a[4] * y.T2 / 3. + a[5] * y.T3 / 4. +
+                     a[6] * y.T4 / 5. + a[8] / y.T;
+    const double r = -a[0] / y.T2 / 2. - a[1] / y.T + a[2] * y.logT + a[3] * y.T + a[4] * y.T2 / 2. + a[5] * y.T3 / 3. +
+                     a[6] * y.T4 / 4. + a[9];
+    return h - r;
 }
 
-__device__ inline double arrh(double A, double n, double E, double T) {
-    return A * pow(T, n) * exp(-E / T);
+constexpr double LN2_HI = 0x1.62e42fefa39efp-1, LN2_LO = 0x1.abc9e3b39803fp-56;   // ln 2 in two doubles
+
+// log x for normal x > 0 as h + l, from log m = 2 atanh((m - 1) / (m + 1)) with
+// the series in two-double arithmetic (|m - 1| / (m + 1) < 0.172: 16 terms
+// leave 1e-25); once per layer
+__device__ inline void log2d(double x, double &h, double &l) {
+    int e;
+    double m = frexp(x, &e);
+    if (m < 0.70710678118654752) {
+        m *= 2.0;
+        e--;
+    }
+    const double num = m - 1.0, dh = m + 1.0, dl = (1.0 - dh) + m;
+    const double sh = num / dh, sl = (fma(-sh, dh, num) - sh * dl) / dh;
+    const double zh = sh * sh, zl = fma(sh, sh, -zh) + 2.0 * sh * sl;
+    double ph = 0.0, pl = 0.0;
+    for (int j = 15; j >= 0; j--) {
+        const double d = 2 * j + 1, ch = 1.0 / d, cl = fma(-ch, d, 1.0) / d;
+        const double t = ph * zh, tl = fma(ph, zh, -t) + (ph * zl + pl * zh);
+        ph = ch + t;
+        pl = ((ch - ph) + t) + (tl + cl);
+    }
+    const double uh = 2.0 * sh * ph, ul = fma(2.0 * sh, ph, -uh) + 2.0 * (sh * pl + sl * ph);
+    const double eh = e * LN2_HI, el = fma((double)e, LN2_HI, -eh) + e * LN2_LO;
+    const double t = eh + uh, bb = t - eh, tl = ((eh - (t - bb)) + (uh - bb)) + (el + ul);
+    h = t + tl;
+    l = (t - h) + tl;
 }
 
-__global__ void k_rates(int L, int npairs, int ni, const int *__restrict__ kind, const double *__restrict__ par,
-                        const int *__restrict__ rev, const int *__restrict__ reac, const int *__restrict__ prod,
-                        const double *__restrict__ Tco, const double *__restrict__ M, const double *__restrict__ tau,
-                        const double *__restrict__ grt, double *__restrict__ k) {
-    int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= L * npairs) return;
-    int l = idx / npairs, p = idx - l * npairs;
-    double T = Tco[l], m = M[l];
-    const double *pa = par + 8 * p;
-    double kf;
-    switch (kind[p]) {
-    case VK_KIND_ARRH:
-    case VK_KIND_K0:
-        kf = arrh(pa[0], pa[1], pa[2], T);
-        break;
-    case VK_KIND_LIND: {
-        double k0 = arrh(pa[0], pa[1], pa[2], T);
-        double kinf = arrh(pa[3], pa[4], pa[5], T);
-        kf = k0 / (1 + k0 * m / kinf);
-        break;
+// c exp(t + lo) for |t| < 700, |lo| << 1: t = k ln 2 + r, the exponential's
+// series to r^13 / 13! (|r| < 0.35: 4e-18 left out)
+__device__ inline double mul_exp(double c, double t, double lo) {
+    const double k = rint(t * 1.4426950408889634);
+    const double r = fma(-k, LN2_HI, t) + fma(-k, LN2_LO, lo);
+    double q = 1. / 6227020800.;
+    q = fma(q, r, 1. / 479001600.);
+    q = fma(q, r, 1. / 39916800.);
+    q = fma(q, r, 1. / 3628800.);
+    q = fma(q, r, 1. / 362880.);
+    q = fma(q, r, 1. / 40320.);
+    q = fma(q, r, 1. / 5040.);
+    q = fma(q, r, 1. / 720.);
+    q = fma(q, r, 1. / 120.);
+    q = fma(q, r, 1. / 24.);
+    q = fma(q, r, 1. / 6.);
+    q = fma(q, r, 0.5);
+    const double e = fma(q, r * r, r);
+    return ldexp(fma(c, e, c), (int)k);
+}
+
+constexpr double EXP_FAST = 650.0;                    // |exponents| of the fast paths
+__device__ inline bool rate_normal(double k) { return fabs(k) > 1e-280 && fabs(k) < 1e280; }
+
+// A T^n exp(-E/T)
+__device__ inline double arrh(double A, double n, double E, const LayerRate &y) {
+    const double q = E * y.rT, ql = fma(-q, y.T, E) * y.rT;              // E/T = q + ql
+    const double h = n * y.lh, hl = fma(n, y.lh, -h) + n * y.ll;         // n log T = h + hl
+    const double t = h - q, bb = t - h, tl = (h - (t - bb)) - (q + bb);  // h - q = t + tl
+    const bool in = fabs(h) < EXP_FAST && fabs(q) < EXP_FAST && fabs(t) < EXP_FAST;   // false for NaN
+    const double k = in ? mul_exp(A, t, tl + (hl - ql)) : 0.0;
+    if (rate_normal(k)) return k;
+    return A * pow(y.T, n) * exp(-E / y.T);
+}
+
+__global__ void __launch_bounds__(BLK, 4) k_rates(int L, int LG, int npairs, int ni, const int *__restrict__ kind,
+                                               const double *__restrict__ par, const int *__restrict__ rev,
+                                               const int *__restrict__ reac, const int *__restrict__ prod,
+                                               const double *__restrict__ nasa9, const double *__restrict__ Tco,
+                                               const double *__restrict__ M, const double *__restrict__ tau,
+                                               double *__restrict__ k) {
+    __shared__ LayerRate lay[RATE_LAYERS];
+    __shared__ double gl[RATE_LAYERS][VK_NI_MAX + 1];    // the last entry: no species, 0
+    const int l0 = blockIdx.x * LG, nl = min(LG, L - l0);
+    if ((int)threadIdx.x < nl) {
+        LayerRate y;
+        const int l = l0 + threadIdx.x;
+        y.T = Tco[l];
+        y.rT = 1.0 / y.T;
+        y.lh = y.ll = nan("");
+        if (y.T > 1e-300 && y.T < 1e300) log2d(y.T, y.lh, y.ll);
+        y.M = M[l];
+        y.emtau = exp(-(tau ? tau[l] : 0.0));
+        y.x = CORR * y.T;
+        y.rx = 1.0 / y.x;
+        y.logT = log(y.T);
+        y.T2 = y.T * y.T;
+        y.T3 = pow(y.T, 3.0);
+        y.T4 = pow(y.T, 4.0);
+        lay[threadIdx.x] = y;
+        gl[threadIdx.x][ni] = 0.0;
     }
-    case VK_KIND_TROE: {
-        double k0 = arrh(pa[0], pa[1], pa[2], T);
-        double kinf = arrh(pa[3], pa[4], pa[5], T);
-        double Fc = pa[6];
-        double nn = 0.75 - 1.27 * log(Fc);
-        double q = log(k0 * m / kinf) / nn;
-        double ff = exp(log(Fc) / (1. + q * q));
-        kf = k0 / (1 + k0 * m / kinf) * ff;
-        break;
+    __syncthreads();
+    for (int q = threadIdx.x; q < nl * ni; q += BLK) {
+        const int a = q / ni, s = q - a * ni;
+        gl[a][s] = g_layer(lay[a], nasa9 + 20 * s);
     }
-    case VK_KIND_PHOTO:
-        kf = pa[7] * exp(-(tau ? tau[l] : 0.0));
-        break;
-    case VK_KIND_CH3OH: {
-        double k0 = 1.932E3 * pow(T, -9.88) * exp(-7544. / T) + 5.109E-11 * pow(T, -6.25) * exp(-1433. / T);
-        double kinf = 1.031E-10 * pow(T, -0.018) * exp(16.74 / T);
-        double Fc = 0.1855 * exp(-T / 155.8) + 0.8145 * exp(-T / 1675.) + exp(-4531. / T);
-        double nn = 0.75 - 1.27 * log(Fc);
-        double q = log(k0 * m / kinf) / nn;
-        double ff = exp(log(Fc) / (1. + q * q));
-        kf = k0 / (1 + k0 * m / kinf) * ff;
-        break;
-    }
-    default:
-        kf = 0.0;
-    }
-    double kr = 0.0;
-    if (rev[p]) {
-        // K = exp(-(-g_r1 - g_r2 + g_p1 + g_p2)) * (corr T)^(n_r - n_p)  (make_chem_funs.py:568-580)
-        const double *g = grt + (size_t)l * ni;
-        double acc = 0.0;
-        bool first = true;
-        int nre = 0, npr = 0;
+    __syncthreads();
+    for (int p = blockIdx.y * BLK + threadIdx.x; p < npairs; p += BLK * gridDim.y) {
+        double pa[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) pa[q] = par[8 * p + q];
+        const int kd = kind[p], rv = rev[p];
+        const int narrh = kd == VK_KIND_ARRH || kd == VK_KIND_K0 ? 1 : (kd == VK_KIND_LIND || kd == VK_KIND_TROE ? 2 : 0);
+        int sr[4], sp[4], dn = 0;
+#pragma unroll
         for (int q = 0; q < 4; q++) {
-            int t = reac[4 * p + q];
-            if (t >= 0) {
-                t = VK_IX(t, ni, VK_SITE_SPECIES);
-                acc = first ? -1 * g[t] : acc - 1 * g[t];
-                first = false;
-                nre++;
+            const int r = reac[4 * p + q], o = prod[4 * p + q];
+            sr[q] = r >= 0 ? VK_IX(r, ni, VK_SITE_SPECIES) : ni;
+            sp[q] = o >= 0 ? VK_IX(o, ni, VK_SITE_SPECIES) : ni;
+            dn += (r >= 0) - (o >= 0);
+        }
+        for (int a = 0; a < nl; a++) {
+            const LayerRate &y = lay[a];
+            const double T = y.T, m = y.M;
+            // the one or two Arrhenius expressions of the pair, in a loop: one
+            // copy of the code
+            double k0 = 0.0, kinf = 0.0;
+#pragma unroll 1
+            for (int h = 0; h < narrh; h++) {
+                const double v = arrh(h ? pa[3] : pa[0], h ? pa[4] : pa[1], h ? pa[5] : pa[2], y);
+                k0 = h ? k0 : v;
+                kinf = h ? v : kinf;
             }
-        }
-        for (int q = 0; q < 4; q++) {
-            int t = prod[4 * p + q];
-            if (t >= 0) {
-                t = VK_IX(t, ni, VK_SITE_SPECIES);
-                acc = first ? 1 * g[t] : acc + 1 * g[t];
-                first = false;
-                npr++;
+            double kf;
+            switch (kd) {
+            case VK_KIND_ARRH:
+            case VK_KIND_K0:
+                kf = k0;
+                break;
+            case VK_KIND_LIND:
+                kf = k0 / (1 + k0 * m / kinf);
+                break;
+            case VK_KIND_CH3OH:
+                k0 = 1.932E3 * pow(T, -9.88) * exp(-7544. / T) + 5.109E-11 * pow(T, -6.25) * exp(-1433. / T);
+                kinf = 1.031E-10 * pow(T, -0.018) * exp(16.74 / T);
+                [[fallthrough]];
+            case VK_KIND_TROE: {
+                const double Fc = kd == VK_KIND_TROE
+                                      ? pa[6]
+                                      : 0.1855 * exp(-T / 155.8) + 0.8145 * exp(-T / 1675.) + exp(-4531. / T);
+                double nn = 0.75 - 1.27 * log(Fc);
+                double q = log(k0 * m / kinf) / nn;
+                double ff = exp(log(Fc) / (1. + q * q));
+                kf = k0 / (1 + k0 * m / kinf) * ff;
+                break;
             }
+            case VK_KIND_PHOTO:
+                kf = pa[7] * y.emtau;
+                break;
+            default:
+                kf = 0.0;
+            }
+            double kr = 0.0;
+            if (rv) {
+                // K = exp(-(-g_r1 - g_r2 + g_p1 + g_p2)) * (corr T)^(n_r - n_p)  (make_chem_funs.py:568-580)
+                double acc = 0.0;
+#pragma unroll
+                for (int q = 0; q < 4; q++) acc -= gl[a][sr[q]];
+#pragma unroll
+                for (int q = 0; q < 4; q++) acc += gl[a][sp[q]];
+                if (fabs(acc) < EXP_FAST && dn >= -1 && dn <= 1)
+                    kr = mul_exp(kf, acc, 0.0) * (dn == 0 ? 1.0 : (dn == 1 ? y.rx : y.x));
+                if (!rate_normal(kr)) {
+                    double K = exp(-acc);
+                    if (dn != 0) {
+                        double f;
+                        if (dn == 1) f = y.x;
+                        else if (dn == -1) f = 1.0 / y.x;
+                        else if (dn == 2) f = y.x * y.x;
+                        else f = pow(y.x, (double)dn);
+                        K = K * f;
+                    }
+                    kr = kf / K;
+                }
+            }
+            double *out = k + 2 * ((size_t)(l0 + a) * npairs + p);
+            out[0] = kf;
+            out[1] = kr;
         }
-        double K = exp(-(acc));
-        int dn = nre - npr;
-        if (dn != 0) {
-            double x = CORR * T;
-            double f;
-            if (dn == 1) f = x;
-            else if (dn == -1) f = 1.0 / x;
-            else if (dn == 2) f = x * x;
-            else f = pow(x, (double)dn);
-            K = K * f;
-        }
-        kr = kf / K;
     }
-    k[(size_t)l * 2 * npairs + 2 * p] = kf;
-    k[(size_t)l * 2 * npairs + 2 * p + 1] = kr;
 }
 
 // ---------------------------------------------------------------------------
@@ -481,16 +591,17 @@ static size_t jac_smem(const vk_plan *p) { return sizeof(double) * (4 * VK_NI_MA
 
 extern "C" int vk_rates(const vk_plan *plan, const vk_columns *cols, const vk_atm *atm, double *d_k, void *stream) {
     if (!plan || !cols || !atm || !d_k) return VK_EINVAL;
-    int L = cols->L;
-    double *grt = nullptr;
-    VK_CHECK(hipMallocAsync((void **)&grt, sizeof(double) * (size_t)L * plan->ni, S(stream)));
-    int n1 = L * plan->ni;
-    hipLaunchKernelGGL(k_grt, dim3((n1 + 255) / 256), dim3(256), 0, S(stream), L, plan->ni, atm->Tco, plan->nasa9, grt);
-    int n2 = L * plan->npairs;
-    hipLaunchKernelGGL(k_rates, dim3((n2 + 255) / 256), dim3(256), 0, S(stream), L, plan->npairs, plan->ni,
-                       plan->kind, plan->par, plan->rev, plan->reac, plan->prod, atm->Tco, atm->M, atm->tau, grt, d_k);
+    const int L = cols->L, cu = vk_device_cus();
+    // layers per workgroup: the most (their pairs' parameters are read once)
+    // that still leave eight workgroups per CU; below that one layer each, and
+    // its pairs over several workgroups
+    int LG = RATE_LAYERS;
+    while (LG > 1 && L < 8 * cu * LG) LG /= 2;
+    const int split = LG > 1 ? 1 : (plan->npairs + BLK - 1) / BLK;
+    hipLaunchKernelGGL(k_rates, dim3((L + LG - 1) / LG, split), dim3(BLK), 0, S(stream), L, LG, plan->npairs, plan->ni,
+                       plan->kind, plan->par, plan->rev, plan->reac, plan->prod, plan->nasa9, atm->Tco, atm->M,
+                       atm->tau, d_k);
     VK_CHECK(hipGetLastError());
-    VK_CHECK(hipFreeAsync(grt, S(stream)));
     return 0;
 }
 

@@ -47,24 +47,6 @@ __device__ inline double pw_sum(const double *a, int n) {
     return 0.0 + (lo + hi);
 }
 
-// NASA9 h/RT and s/R (thermo/gibbs_text.txt:13-18)
-__device__ inline double h_RT(double T, const double *a) {
-    return -a[0] / (T * T) + a[1] * log(T) / T + a[2] + a[3] * T / 2. + a[4] * (T * T) / 3.
-         + a[5] * pow(T, 3.0) / 4. + a[6] * pow(T, 4.0) / 5. + a[8] / T;
-}
-__device__ inline double s_R(double T, const double *a) {
-    return -a[0] / (T * T) / 2. - a[1] / T + a[2] * log(T) + a[3] * T + a[4] * (T * T) / 2.
-         + a[5] * pow(T, 3.0) / 3. + a[6] * pow(T, 4.0) / 4. + a[9];
-}
-// g/RT: low set below 1000 K, high set at and above (chem_funs.py:2789-2792)
-__device__ inline double g_RT(double T, const double *a20) {
-    double glo = h_RT(T, a20) - s_R(T, a20);
-    double ghi = h_RT(T, a20 + 10) - s_R(T, a20 + 10);
-    double mlo = (T < 1000.0) ? 1.0 : 0.0;
-    double mhi = (T >= 1000.0) ? 1.0 : 0.0;
-    return mlo * glo + mhi * ghi;
-}
-
 // Column-local view of the atmosphere arrays.
 struct ColAtm {
     const double *Kzz, *dzi, *Ti, *Hpi, *Tco, *g, *Dzz;
