@@ -293,11 +293,12 @@ __device__ inline double pair_rate(const int4 *reac, const int4 *prod, const dou
     return a - b;
 }
 
-// d/dy_sp of kcol * prod(terms)
-__device__ inline double dside(int4 t4, double kcol, const double *yl, double m, int sp, bool &any, int ni) {
+// d/dy_sp of kcol * prod(terms), yl[LG s] the amount of species s
+template <int LG>
+__device__ inline double dside(int4 t4, double kcol, const double *yl, double m, int sp, int ni) {
     const int t[4] = {t4.x, t4.y, t4.z, t4.w};
     double tot = 0.0;
-    any = false;
+    bool any = false;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         if (t[q] != sp) continue;
@@ -305,7 +306,7 @@ __device__ inline double dside(int4 t4, double kcol, const double *yl, double m,
 #pragma unroll
         for (int q2 = 0; q2 < 4; q2++) {
             if (q2 == q || t[q2] == -2) continue;
-            acc = acc * (t[q2] == -1 ? m : yl[VK_IX(t[q2], ni, VK_SITE_SPECIES)]);
+            acc = acc * (t[q2] == -1 ? m : yl[LG * VK_IX(t[q2], ni, VK_SITE_SPECIES)]);
         }
         tot = any ? tot + acc : acc;
         any = true;
@@ -397,124 +398,128 @@ __global__ void __launch_bounds__(BLK) k_rhs(
 
 // ---------------------------------------------------------------------------
 // Jacobian blocks (mode 0: J = d chemdf/dy) or Ros2 lhs blocks (mode 1:
-// D = c0 I - J - J_diff, Lsub, Usup), one workgroup per layer
+// D = c0 I - J - J_diff, Lsub, Usup), one workgroup per LG layers.
+//
+// Bound by instructions and the table reads, not by the block it writes: the
+// tables (38 KB of slots, 70 KB of entries for 93 species and 620 pairs) are
+// laid out so that a slot is two products of three looked-up amounts and an
+// entry's first two terms come with it, and with two layers a workgroup reads
+// them once for both (a slot's values of the layers side by side in LDS).
+// 93 species, 620 pairs: 36 000 layers 1695 -> 1310 us (1435 with one layer a
+// workgroup; the vector cache waits on L2 for four fifths of it, the 2.7 GB of
+// sectors it touches take 0.4 ms), 1700 layers 131 -> 87 us, 150 layers
+// 39 -> 22 us.
 // ---------------------------------------------------------------------------
 
 // The diagonal of a layer's lhs block after c0 - J: the diffusion terms in
 // the reference's order.  xmode 1: the escape term first (top layer, _vm
 // operators, op.py:2101-2107); xmode 2: the deposition velocity last (bottom
 // layer, op.py:2029).
-__device__ __forceinline__ double lhs_diag(double val, int i, int mol, const double *dg0, const double *dg1,
-                                           const double *dgx, int xmode) {
-    if (xmode == 1) val = val - dgx[i];
-    val = val - dg0[i];
-    if (mol) val = val - dg1[i];
-    if (xmode == 2) val = val - dgx[i];
-    return val;
+struct LhsDiag {
+    double c0;
+    int xmode, mol;
+    const double *dg0, *dg1, *dgx;       // per species
+    __device__ __forceinline__ double operator()(double val, int i) const {
+        val = c0 + val;
+        if (xmode == 1) val = val - dgx[i];
+        val = val - dg0[i];
+        if (mol) val = val - dg1[i];
+        if (xmode == 2) val = val - dgx[i];
+        return val;
+    }
+};
+
+// J += (or =) a packed term, for each layer
+template <int LG>
+__device__ __forceinline__ void add_term(double (&J)[LG], bool first, int t, const double *dv, int nslot) {
+    const double c = vk_jac_coef(t);
+    const double *d = dv + LG * VK_IX(vk_jac_slot(t), nslot, VK_SITE_SLOT);
+#pragma unroll
+    for (int a = 0; a < LG; a++) J[a] = first ? c * d[a] : J[a] + c * d[a];
 }
 
-// one entry of the lhs (mode 1) or of the Jacobian (mode 0): its terms in order
-__device__ __forceinline__ void jac_entry(int q, const int4 *__restrict__ jac_ent, const int *__restrict__ jac_tp,
-                                          const double *dv, int ni, int njac, int nslot, int mode, int mol, double c0,
-                                          const double *dg0, const double *dg1, const double *dgx, int xmode,
-                                          double *__restrict__ Dl) {
-    const int4 en = jac_ent[q];           // (dense index, first term, end of terms, row)
-    double J = 0.0;
-    if (en.z > en.y) {
-        const int t = jac_tp[VK_IX(en.y, njac, VK_SITE_TERM)];
-        J = vk_jac_coef(t) * dv[VK_IX(vk_jac_slot(t), nslot, VK_SITE_SLOT)];
-        // terms in order; four loads in flight per round
-        for (int u = en.y + 1; u < en.z; u += 4) {
-            const int t0 = jac_tp[VK_IX(u, njac, VK_SITE_TERM)];
-            const int t1 = u + 1 < en.z ? jac_tp[VK_IX(u + 1, njac, VK_SITE_TERM)] : t0;
-            const int t2 = u + 2 < en.z ? jac_tp[VK_IX(u + 2, njac, VK_SITE_TERM)] : t0;
-            const int t3 = u + 3 < en.z ? jac_tp[VK_IX(u + 3, njac, VK_SITE_TERM)] : t0;
-            J = J + vk_jac_coef(t0) * dv[VK_IX(vk_jac_slot(t0), nslot, VK_SITE_SLOT)];
-            if (u + 1 < en.z) J = J + vk_jac_coef(t1) * dv[VK_IX(vk_jac_slot(t1), nslot, VK_SITE_SLOT)];
-            if (u + 2 < en.z) J = J + vk_jac_coef(t2) * dv[VK_IX(vk_jac_slot(t2), nslot, VK_SITE_SLOT)];
-            if (u + 3 < en.z) J = J + vk_jac_coef(t3) * dv[VK_IX(vk_jac_slot(t3), nslot, VK_SITE_SLOT)];
-        }
+template <int LG>
+__global__ void __launch_bounds__(BLK *LG, 4) k_jac_lhs(
+    int L, int ni, int npairs, int nslot, int nlight, int nheavy, int njac, const int *__restrict__ off,
+    const int *__restrict__ layer_col, const int *__restrict__ reac, const int *__restrict__ prod,
+    const int4 *__restrict__ slot_tab, const int4 *__restrict__ jac_ent, const int4 *__restrict__ jac_light,
+    const int *__restrict__ jac_emap, const int *__restrict__ jac_tp, const double *__restrict__ ms,
+    const double *__restrict__ alpha, vk_atm atm, const double *__restrict__ y, const double *__restrict__ k,
+    const double *__restrict__ M, int mode, int mol, const double *__restrict__ dtc, const double *__restrict__ ysum,
+    const vk_colstate *__restrict__ st, double *__restrict__ D, double *__restrict__ Lsub, double *__restrict__ Usup,
+    int write_zeros) {
+    extern __shared__ __align__(16) double smem[];
+    double *dv = smem;                                 // nslot x LG
+    double *yl = dv + LG * nslot;                      // (ni + 2) x LG: amounts, then M and one
+    double *dg = yl + LG * (VK_NI_MAX + 2);            // LG x 3 VK_NI_MAX: terms of the diagonal, per species
+    const int l0 = blockIdx.x * LG, nn = ni * ni;
+    LayerCtx x[LG];
+    bool on[LG], any = false;
+#pragma unroll
+    for (int a = 0; a < LG; a++) {
+        x[a] = layer_ctx(off, layer_col, min(l0 + a, L - 1));
+        on[a] = l0 + a < L && !(st && st[x[a].c].done);
+        any = any || on[a];
     }
-    const int ex = VK_IX(en.x, ni * ni, VK_SITE_DENSE);
-    if (mode == 0) {
-        Dl[ex] = J;
-        return;
-    }
-    const int i = en.w;
-    double val = -J;
-    if (ex == i * ni + i) val = lhs_diag(c0 + val, i, mol, dg0, dg1, dgx, xmode);
-    Dl[ex] = val;
-}
-
-__global__ void __launch_bounds__(BLK) k_jac_lhs(
-    int ni, int npairs, int nslot, int nent, int njac, const int *__restrict__ off, const int *__restrict__ layer_col,
-    const int *__restrict__ reac, const int *__restrict__ prod, const int *__restrict__ slot_pair,
-    const int *__restrict__ slot_sp, const int4 *__restrict__ jac_ent, const int *__restrict__ jac_emap, int nheavy,
-    const int *__restrict__ jac_tp,
-    const double *__restrict__ ms, const double *__restrict__ alpha, vk_atm atm, const double *__restrict__ y,
-    const double *__restrict__ k, const double *__restrict__ M, int mode, int mol, const double *__restrict__ dtc,
-    const double *__restrict__ ysum, const vk_colstate *__restrict__ st, double *__restrict__ D,
-    double *__restrict__ Lsub, double *__restrict__ Usup, int write_zeros) {
-    extern __shared__ double smem[];
-    double *yl = smem;                       // ni
-    double *dg0 = smem + VK_NI_MAX;          // diffusion terms of the diagonal, per species
-    double *dg1 = smem + 2 * VK_NI_MAX;
-    double *dgx = smem + 3 * VK_NI_MAX;      // escape (top) or deposition (bottom) term
-    double *dv = smem + 4 * VK_NI_MAX;       // nslot
-    const int l = blockIdx.x;
-    LayerCtx x = layer_ctx(off, layer_col, l);
-    if (st && st[x.c].done) return;
-    const double *yrow = y + (size_t)l * ni;
-    for (int i = threadIdx.x; i < ni; i += blockDim.x) yl[i] = yrow[i];
+    if (!any) return;
+    for (int q = threadIdx.x; q < ni + 2; q += BLK * LG)
+#pragma unroll
+        for (int a = 0; a < LG; a++)
+            yl[LG * q + a] = q < ni ? y[(size_t)x[a].l * ni + q] : (q == ni ? M[x[a].l] : 1.0);
     __syncthreads();   // the slot derivatives read yl
-    const int nn = ni * ni;
-    double *Dl = D + (size_t)l * nn;
-    const double *kl = k + (size_t)l * 2 * npairs;
-    const double m = M[l];
-    // slot derivatives: JS slots per thread per round, every load of a round
-    // (slot -> pair -> the pair's sides and rates, three loads deep) issued
-    // before its arithmetic
-    constexpr int JS = 4;
-    for (int s0 = threadIdx.x; s0 < nslot; s0 += JS * blockDim.x) {
-        int p[JS], sp[JS];
+    for (int s = threadIdx.x; s < nslot; s += BLK * LG) {
+        const int4 e = slot_tab[s];
+        const int p = VK_IX(e.x, npairs, VK_SITE_SLOTPAIR);
+        double kf[LG], kb[LG], d[LG];
 #pragma unroll
-        for (int u = 0; u < JS; u++) {
-            const int s = s0 + u * blockDim.x;
-            p[u] = s < nslot ? VK_IX(slot_pair[s], npairs, VK_SITE_SLOTPAIR) : 0;
-            sp[u] = s < nslot ? slot_sp[s] : 0;
+        for (int a = 0; a < LG; a++) {
+            const double *kl = k + ((size_t)x[a].l * npairs + p) * 2;
+            kf[a] = kl[0];
+            kb[a] = kl[1];
         }
-        int4 rt[JS], pt[JS];
-        double kf[JS], kb[JS];
+        auto product = [&](int side, const double (&kc)[LG], double sign) {
+            const double *f0 = yl + LG * VK_IX(side & 255, ni + 2, VK_SITE_SPECIES);
+            const double *f1 = yl + LG * VK_IX(side >> 8 & 255, ni + 2, VK_SITE_SPECIES);
+            const double *f2 = yl + LG * VK_IX(side >> 16 & 255, ni + 2, VK_SITE_SPECIES);
 #pragma unroll
-        for (int u = 0; u < JS; u++) {
-            rt[u] = ((const int4 *)reac)[p[u]];
-            pt[u] = ((const int4 *)prod)[p[u]];
-            kf[u] = kl[2 * p[u]];
-            kb[u] = kl[2 * p[u] + 1];
-        }
+            for (int a = 0; a < LG; a++) {
+                const double v = kc[a] * f0[a] * f1[a] * f2[a];
+                d[a] = sign > 0 ? (side >> 24 ? v : 0.0) : d[a] - (side >> 24 ? v : 0.0);
+            }
+        };
+        product(e.y, kf, 1.0);
+        product(e.z, kb, -1.0);
+        if (((e.y | e.z) >> 24) & 2) {
+            const int4 rt = ((const int4 *)reac)[p], pt = ((const int4 *)prod)[p];
 #pragma unroll
-        for (int u = 0; u < JS; u++) {
-            const int s = s0 + u * blockDim.x;
-            if (s < nslot) {
-                bool a1, a2;
-                const double dr = dside(rt[u], kf[u], yl, m, sp[u], a1, ni);
-                const double dp = dside(pt[u], kb[u], yl, m, sp[u], a2, ni);
-                dv[s] = (a1 ? dr : 0.0) - (a2 ? dp : 0.0);
+            for (int a = 0; a < LG; a++) {
+                const double m = yl[LG * ni + a];
+                d[a] = dside<LG>(rt, kf[a], yl + a, m, e.w, ni) - dside<LG>(pt, kb[a], yl + a, m, e.w, ni);
             }
         }
+#pragma unroll
+        for (int a = 0; a < LG; a++) dv[LG * s + a] = d[a];
     }
-    double c0 = 0.0;
-    int xmode = 0;
-    if (mode == 1) {
+    LhsDiag diag[LG];
+#pragma unroll
+    for (int a = 0; a < LG; a++) {
+        double *dg0 = dg + 3 * VK_NI_MAX * a, *dg1 = dg0 + VK_NI_MAX, *dgx = dg1 + VK_NI_MAX;
+        diag[a] = {0.0, 0, mol, dg0, dg1, dgx};
+        if (mode != 1) continue;
         // diffusion part of the lhs (op.py:2012-2040): once per species
-        c0 = 1. / (R_ROS * dtc[x.c]);
+        const LayerCtx &xa = x[a];
+        diag[a].c0 = 1. / (R_ROS * dtc[xa.c]);
         double ysm, ys0, ysp;
-        ysum_around(ysum, x, ysm, ys0, ysp);
-        ColAtm ca = col_atm(atm, x.c, x.off, x.nz, ni);
-        if (x.j == 0 && ca.use_bot) xmode = 2;
-        else if (x.j == x.nz - 1 && ca.vm && mol && atm.top_flux && esc_any(atm)) xmode = 1;
-        for (int i = threadIdx.x; i < ni; i += blockDim.x) {
-            LhsDiff r = lhs_diff(ca, x.j, i, ysm, ys0, ysp, ms[i], alpha[i], mol != 0);
+        ysum_around(ysum, xa, ysm, ys0, ysp);
+        ColAtm ca = col_atm(atm, xa.c, xa.off, xa.nz, ni);
+        int xmode = 0;
+        if (xa.j == 0 && ca.use_bot) xmode = 2;
+        else if (xa.j == xa.nz - 1 && ca.vm && mol && atm.top_flux && esc_any(atm)) xmode = 1;
+        diag[a].xmode = xmode;
+        // each layer's species on threads of their own
+        for (int i = (int)threadIdx.x - BLK * a; i < ni; i += BLK * LG) {
+            if (i < 0) continue;
+            LhsDiff r = lhs_diff(ca, xa.j, i, ysm, ys0, ysp, ms[i], alpha[i], mol != 0);
             dg0[i] = r.d0;
             dg1[i] = r.d1;
             if (xmode == 2) {
@@ -522,60 +527,77 @@ __global__ void __launch_bounds__(BLK) k_jac_lhs(
             } else if (xmode == 1) {
                 // diff_lim = top_flux / y for escaping species with y > 0 (no 1/dzi, as there)
                 double e = 0.0;
-                if (((atm.esc[i >> 5] >> (i & 31)) & 1u) && yrow[i] > 0)
-                    e = 0.0 + atm.top_flux[(size_t)x.c * ni + i] / yrow[i];
+                if (((atm.esc[i >> 5] >> (i & 31)) & 1u) && yl[LG * i + a] > 0)
+                    e = 0.0 + atm.top_flux[(size_t)xa.c * ni + i] / yl[LG * i + a];
                 dgx[i] = e;
             }
             double u = 0.0, lo = 0.0;
             if (r.has_u) { u = 0.0 - r.u0; if (r.has_mol) u = u - r.u1; }
             if (r.has_l) { lo = 0.0 - r.l0; if (r.has_mol) lo = lo - r.l1; }
-            if (blockIdx.y == 0) {
-                Usup[(size_t)l * ni + i] = u;
-                Lsub[(size_t)l * ni + i] = lo;
+            if (blockIdx.y == 0 && on[a]) {
+                Usup[(size_t)xa.l * ni + i] = u;
+                Lsub[(size_t)xa.l * ni + i] = lo;
             }
         }
     }
     __syncthreads();
     // Every dense entry is written once (the structural zeros only with
-    // write_zeros: the integrator clears its blocks once and skips them).
-    // Entries with at most JAC_LIGHT
-    // terms (and the structural zeros) in one coalesced pass over the dense
-    // index; the few long term lists (jac_ent[0, nheavy): the list is sorted
-    // by term count) by their own threads alongside.  With few layers the
-    // entries of a layer are split over the grid's y dimension (each
-    // workgroup forms the layer's shared terms itself).
-    const int e0 = threadIdx.x + blockIdx.y * blockDim.x, es = blockDim.x * gridDim.y;
-    for (int q = e0; q < nheavy; q += es)
-        jac_entry(q, jac_ent, jac_tp, dv, ni, njac, nslot, mode, mol, c0, dg0, dg1, dgx, xmode, Dl);
-#pragma unroll 4
-    for (int e = e0; e < nn; e += es) {
-        // (first term << 4 | term count), -1: structural zero, -2: long term list
-        const int code = jac_emap[e];
-        if (code == -2 || (code == -1 && !write_zeros)) continue;
-        double val = 0.0;
-        if (code >= 0) {
-            const int u0 = code >> 4, nt = code & 15;
-            double J = 0.0;
-            if (nt > 0) {
-                // only the entry's own terms are loaded (all issued before the sums)
-                int t[VK_JAC_LIGHT];
+    // write_zeros: the integrator clears its blocks once and skips them): the
+    // few long term lists (jac_ent[0, nheavy): the list is sorted by term
+    // count) by threads of their own, the others in one nearly coalesced pass
+    // in the order of the dense index.  With few layers the entries of a
+    // layer are split over the grid's y dimension (each workgroup forms the
+    // layer's shared terms itself).
+    auto store = [&](int e, const double (&J)[LG], bool dg) {
+        e = VK_IX(e, nn, VK_SITE_DENSE);
 #pragma unroll
-                for (int m = 0; m < VK_JAC_LIGHT; m++) t[m] = m < nt ? jac_tp[VK_IX(u0 + m, njac, VK_SITE_TERM)] : 0;
-                J = vk_jac_coef(t[0]) * dv[VK_IX(vk_jac_slot(t[0]), nslot, VK_SITE_SLOT)];
-#pragma unroll
-                for (int m = 1; m < VK_JAC_LIGHT; m++)
-                    if (m < nt) J = J + vk_jac_coef(t[m]) * dv[VK_IX(vk_jac_slot(t[m]), nslot, VK_SITE_SLOT)];
+        for (int a = 0; a < LG; a++) {
+            double val = J[a];
+            if (mode) {
+                val = -val;
+                if (dg) val = diag[a](val, e / (ni + 1));
             }
-            if (mode == 0) {
-                val = J;
-            } else {
-                const int i = e / ni;
-                val = -J;
-                if (e == i * ni + i) val = lhs_diag(c0 + val, i, mol, dg0, dg1, dgx, xmode);
-            }
+            if (on[a]) D[(size_t)x[a].l * nn + e] = val;
         }
-        Dl[e] = val;
+    };
+    const int e0 = threadIdx.x + blockIdx.y * BLK * LG, es = BLK * LG * gridDim.y;
+    for (int q = e0; q < nheavy; q += es) {
+        const int4 en = jac_ent[q];       // (dense index, first term, end of terms, row)
+        double J[LG];
+        add_term<LG>(J, true, jac_tp[VK_IX(en.y, njac, VK_SITE_TERM)], dv, nslot);
+        // terms in order; eight loads in flight per round
+        int u = en.y + 1;
+        for (; u + 8 <= en.z; u += 8) {
+            int t[8];
+#pragma unroll
+            for (int m = 0; m < 8; m++) t[m] = jac_tp[VK_IX(u + m, njac, VK_SITE_TERM)];
+#pragma unroll
+            for (int m = 0; m < 8; m++) add_term<LG>(J, false, t[m], dv, nslot);
+        }
+        for (; u < en.z; u++) add_term<LG>(J, false, jac_tp[VK_IX(u, njac, VK_SITE_TERM)], dv, nslot);
+        store(en.x, J, en.x == en.w * (ni + 1));
     }
+#pragma unroll 2
+    for (int q = e0; q < nlight; q += es) {
+        const int4 en = jac_light[q];
+        const int nt = en.x >> 16 & 15;
+        int t[VK_JAC_LIGHT];
+#pragma unroll
+        for (int m = 2; m < VK_JAC_LIGHT; m++) t[m] = m < nt ? jac_tp[VK_IX(en.y + m, njac, VK_SITE_TERM)] : 0;
+        double J[LG] = {};
+        if (nt > 0) add_term<LG>(J, true, en.z, dv, nslot);
+        if (nt > 1) add_term<LG>(J, false, en.w, dv, nslot);
+#pragma unroll
+        for (int m = 2; m < VK_JAC_LIGHT; m++)
+            if (m < nt) add_term<LG>(J, false, t[m], dv, nslot);
+        store(en.x & 0xffff, J, en.x >> 20);
+    }
+    if (write_zeros)
+        for (int e = e0; e < nn; e += es)
+            if (jac_emap[e] < 0)
+#pragma unroll
+                for (int a = 0; a < LG; a++)
+                    if (on[a]) D[(size_t)x[a].l * nn + e] = 0.0;
 }
 
 }  // namespace
@@ -587,7 +609,9 @@ __global__ void __launch_bounds__(BLK) k_jac_lhs(
 static inline hipStream_t S(void *s) { return (hipStream_t)s; }
 
 static size_t rhs_smem(const vk_plan *p) { return sizeof(double) * (VK_NI_MAX + (size_t)p->npairs); }
-static size_t jac_smem(const vk_plan *p) { return sizeof(double) * (4 * VK_NI_MAX + (size_t)p->nslot); }
+static size_t jac_smem(const vk_plan *p, int layers) {
+    return sizeof(double) * layers * (4 * VK_NI_MAX + 2 + (size_t)p->nslot);
+}
 
 extern "C" int vk_rates(const vk_plan *plan, const vk_columns *cols, const vk_atm *atm, double *d_k, void *stream) {
     if (!plan || !cols || !atm || !d_k) return VK_EINVAL;
@@ -643,19 +667,21 @@ int vk_launch_jac_lhs(const vk_plan *plan, const vk_columns *cols, const vk_atm 
             if (r) return r;
         }
     }
-    // fewer layers than twice the CUs: split each layer's entries over up to 4 workgroups
-    static const int ncu = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            return 0;
-        return n;
-    }();
-    const int gy = ncu > 0 ? std::max(1, std::min(4, 2 * ncu / std::max(cols->L, 1))) : 1;
-    hipLaunchKernelGGL(k_jac_lhs, dim3(cols->L, gy), dim3(BLK), jac_smem(plan), s, plan->ni, plan->npairs, plan->nslot,
-                       plan->njent, plan->njac, cols->d_off, cols->d_layer_col, plan->reac, plan->prod, plan->slot_pair,
-                       plan->slot_sp, plan->jac_ent, plan->jac_emap, plan->njheavy, plan->jac_tp, plan->ms, plan->alpha, a, y, k, M, mode, mol,
-                       dtc, ysum, st, D, Lsub, Usup, (int)write_zeros);
+    const int ncu = vk_device_cus();
+    auto launch = [&](auto kernel, int layers, int gy) {
+        hipLaunchKernelGGL(kernel, dim3((cols->L + layers - 1) / layers, gy), dim3(BLK * layers), jac_smem(plan, layers),
+                           s, cols->L, plan->ni, plan->npairs, plan->nslot, plan->njlight, plan->njheavy, plan->njac,
+                           cols->d_off, cols->d_layer_col, plan->reac, plan->prod, plan->slot_tab, plan->jac_ent,
+                           plan->jac_light, plan->jac_emap, plan->jac_tp, plan->ms, plan->alpha, a, y, k, M, mode, mol,
+                           dtc, ysum, st, D, Lsub, Usup, (int)write_zeros);
+    };
+    // two layers a workgroup where two such workgroups fit a CU's 160 KB and
+    // every CU still gets several; fewer layers than twice the CUs: each
+    // layer's entries over up to 4 workgroups
+    if (jac_smem(plan, 2) <= 80 * 1024 && cols->L >= 12 * ncu)
+        launch(k_jac_lhs<2>, 2, 1);
+    else
+        launch(k_jac_lhs<1>, 1, ncu > 0 ? std::max(1, std::min(4, 2 * ncu / std::max(cols->L, 1))) : 1);
     VK_CHECK(hipGetLastError());
     return 0;
 }

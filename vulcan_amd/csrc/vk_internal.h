@@ -38,6 +38,28 @@ __host__ __device__ inline int vk_jac_pack(int slot, int coef) { return (slot <<
 __host__ __device__ inline int vk_jac_slot(int w) { return w >> 8; }
 __host__ __device__ inline double vk_jac_coef(int w) { return (double)((int)((unsigned)w << 24) >> 24); }
 
+// an entry of jac_light: dense index, term count, on the diagonal
+static_assert(VK_NI_MAX * VK_NI_MAX <= 1 << 16 && VK_JAC_LIGHT < 16, "fields of vk_light_pack");
+__host__ __device__ inline int vk_light_pack(int e, int nt, bool diag) { return e | nt << 16 | (int)diag << 20; }
+
+// d(side of a pair)/dy_sp as a product: k times the amounts with the indices
+// in the low three bytes (species; ni: M; ni + 1: one), in the side's order.
+// Top byte: 0 the species is not on this side, 1 such a product, 2 neither
+// (a species more than once): summed term by term in the kernel.
+static_assert(VK_NI_MAX + 2 <= 256, "bytes of vk_side_pack");
+inline int vk_side_pack(const int *t, int sp, int ni) {
+    int at = -1, count = 0;
+    for (int q = 0; q < 4; q++) {
+        if (t[q] >= ni || t[q] < -2) return 2 << 24;
+        if (t[q] == sp) { at = q; count++; }
+    }
+    if (count != 1) return count ? 2 << 24 : 0;
+    int f[3] = {ni + 1, ni + 1, ni + 1}, n = 0;
+    for (int q = 0; q < 4; q++)
+        if (q != at && t[q] != -2) f[n++] = t[q] == -1 ? ni : t[q];
+    return 1 << 24 | f[0] | f[1] << 8 | f[2] << 16;
+}
+
 struct vk_plan {
     int ni, npairs, nr, natom, nchem, nslot, njnz, njac;
     int factor_variant;
@@ -45,11 +67,13 @@ struct vk_plan {
     double *par, *nasa9, *atom_mat, *ms, *alpha;
     int *chem_ptr, *chem_pair, *chem_sign;
     int2 *chem_ent;            // (chem_pair, chem_sign) interleaved
-    int *slot_pair, *slot_sp;
     int *jac_map, *jac_ptr, *jac_slot;
     int njent;                 // entries with chemical terms plus the diagonal
     int4 *jac_ent;             // (dense index, first term, end of terms, row), longest term lists first
-    int *jac_emap;             // dense index -> (first term << 4 | term count) of a short list, -1 zero, -2 long list
+    int *jac_emap;             // dense index -> -1 where the block has a structural zero, else 0
+    int njlight;               // entries with at most VK_JAC_LIGHT terms, by dense index:
+    int4 *jac_light;           // (vk_light_pack, first term, its first two packed terms)
+    int4 *slot_tab;            // (pair, vk_side_pack of its reactants and its products, species) of a derivative slot
     int njheavy;               // entries with more than VK_JAC_LIGHT terms (the first ones of jac_ent)
     int *jac_tp;               // packed terms (vk_jac_pack) in jac_coef / jac_slot order
     double *jac_coef;

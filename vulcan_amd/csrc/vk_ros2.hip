@@ -513,12 +513,11 @@ extern "C" int vk_plan_create(const vk_network_desc *n, vk_plan **out) {
     r = r ? r : upload(v, &p->chem_ptr, n->chem_ptr, (size_t)n->ni + 1);
     r = r ? r : upload(v, &p->chem_pair, n->chem_pair, (size_t)n->nchem);
     r = r ? r : upload(v, &p->chem_sign, n->chem_sign, (size_t)n->nchem);
-    r = r ? r : upload(v, &p->slot_pair, n->slot_pair, (size_t)n->nslot);
-    r = r ? r : upload(v, &p->slot_sp, n->slot_sp, (size_t)n->nslot);
     r = r ? r : upload(v, &p->jac_map, n->jac_map, (size_t)n->ni * n->ni);
     r = r ? r : upload(v, &p->jac_ptr, n->jac_ptr, (size_t)n->njnz + 1);
     r = r ? r : upload(v, &p->jac_slot, n->jac_slot, (size_t)n->njac);
     r = r ? r : upload(v, &p->jac_coef, n->jac_coef, (size_t)n->njac);
+    std::vector<int4> light;       // (dense index, first term, end of terms, row)
     if (!r) {
         std::vector<int4> ent;
         for (int e = 0; e < n->ni * n->ni; e++) {
@@ -535,12 +534,12 @@ extern "C" int vk_plan_create(const vk_network_desc *n, vk_plan **out) {
         p->njheavy = 0;
         std::vector<int> emap((size_t)n->ni * n->ni, -1);
         for (int q = 0; q < p->njent; q++) {
-            const int nt = ent[q].z - ent[q].y;
-            if (nt > VK_JAC_LIGHT) p->njheavy = q + 1;
-            emap[ent[q].x] = nt > VK_JAC_LIGHT ? -2 : (ent[q].y << 4) | nt;
+            if (ent[q].z - ent[q].y > VK_JAC_LIGHT) p->njheavy = q + 1;
+            emap[ent[q].x] = 0;
         }
         r = upload(v, &p->jac_ent, ent.data(), ent.size());
         r = r ? r : upload(v, &p->jac_emap, emap.data(), emap.size());
+        light.assign(ent.begin() + p->njheavy, ent.end());
     }
     if (!r) {
         std::vector<int2> ce((size_t)n->nchem);
@@ -557,6 +556,23 @@ extern "C" int vk_plan_create(const vk_network_desc *n, vk_plan **out) {
             else terms[q] = vk_jac_pack(sl, (int)c);
         }
         r = r ? r : upload(v, &p->jac_tp, terms.data(), terms.size());
+        std::sort(light.begin(), light.end(), [](const int4 &x, const int4 &y) { return x.x < y.x; });
+        for (int4 &e : light) {
+            const int u0 = e.y, nt = e.z - e.y;
+            e = make_int4(vk_light_pack(e.x, nt, e.x % n->ni == e.w), u0, nt > 0 ? terms[u0] : 0,
+                          nt > 1 ? terms[u0 + 1] : 0);
+        }
+        p->njlight = (int)light.size();
+        light.push_back(make_int4(0, 0, 0, 0));      // never empty
+        r = r ? r : upload(v, &p->jac_light, light.data(), light.size());
+        std::vector<int4> slots((size_t)n->nslot + 1);
+        for (int q = 0; q < n->nslot; q++) {
+            const int pr = n->slot_pair[q], sp = n->slot_sp[q];
+            const bool ok = pr >= 0 && pr < n->npairs;
+            slots[q] = make_int4(pr, ok ? vk_side_pack(n->reac + 4 * pr, sp, n->ni) : 2 << 24,
+                                 ok ? vk_side_pack(n->prod + 4 * pr, sp, n->ni) : 2 << 24, sp);
+        }
+        r = r ? r : upload(v, &p->slot_tab, slots.data(), slots.size());
     }
     if (r) { vk_plan_destroy(p); return r; }
     *out = p;
