@@ -243,119 +243,37 @@ __global__ void __launch_bounds__(NT) k_bcr_update(int ni, int n, const int4 *__
     slab_store<NBH>(acc2, ni, r0, Ct + j * nn, true, -1.0, nullptr, c0);
 }
 
-__global__ void k_copy_d(long n, const double *__restrict__ a, double *__restrict__ b) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) b[i] = a[i];
-}
+// Solve sweeps: each block's products are split over row groups of 32 (one
+// workgroup each, grid y), so a block's operators are read by several CUs at
+// once; 256 threads, thread t owns row a0 + t % 32 and part h = t / 32 of the
+// b range (chunks of ceil(ni/8) <= CH).  Every operator entry a thread needs
+// is loaded into registers before the first product, and the eight partial
+// sums of a row are combined through LDS in part order.  9 columns of 61
+// to 110 layers, 150 species: a sweep pair 685 -> 217 us against one workgroup
+// per block without loads ahead; one column of 150 layers, 93 species: 9 % of
+// a sweep from loads that no branch splits.
+constexpr int MV_NT = 256, MV_RG = 32, MV_SP = 8;
 
-// Matrix-vector products of the solves: out[a] = sum_b M[a][b] v[b] with M
-// stored transposed (Mt[b][a]), 256 threads: row a = tid % 128 (+128 ...),
-// half h = tid / 128 of the b range, four independent accumulators per
-// thread so that the loads of a row stay in flight; the two halves are
-// combined by the caller through LDS.
-constexpr int BCR_ST = 256;
-
-__device__ __forceinline__ double tmv_part(const double *__restrict__ Mt, const double *v, int ni, int a, int h) {
-    const int hb = (ni + 1) >> 1, b0 = h * hb, b1 = min(ni, b0 + hb);
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-    int b = b0;
-    for (; b + 3 < b1; b += 4) {
-        s0 = fma(Mt[(size_t)b * ni + a], v[b], s0);
-        s1 = fma(Mt[(size_t)(b + 1) * ni + a], v[b + 1], s1);
-        s2 = fma(Mt[(size_t)(b + 2) * ni + a], v[b + 2], s2);
-        s3 = fma(Mt[(size_t)(b + 3) * ni + a], v[b + 3], s3);
-    }
-    for (; b < b1; b++) s0 = fma(Mt[(size_t)b * ni + a], v[b], s0);
-    return (s0 + s1) + (s2 + s3);
-}
-
-// solves: forward reduction r_j -= P_j r_l + Q_j r_r at level s
-__global__ void __launch_bounds__(BCR_ST) k_bcr_fwd(int ni, int n, const int4 *__restrict__ sv, int slot0,
-                                                    const double *__restrict__ P, const double *__restrict__ Q,
-                                                    double *__restrict__ r, const vk_colstate *__restrict__ st) {
-    const int q = blockIdx.x;
-    if (q >= n) return;
-    const int4 e = sv[q];
-    if (st && st[e.w].done) return;
-    const size_t nn = (size_t)ni * ni;
-    const double *Pj = P + (size_t)(slot0 + q) * nn, *Qj = Q + (size_t)(slot0 + q) * nn;
-    __shared__ double rl[VK_NI_MAX], rr[VK_NI_MAX], pp[2][VK_NI_MAX];
-    for (int i = threadIdx.x; i < ni; i += BCR_ST) {
-        rl[i] = e.y >= 0 ? r[(size_t)e.y * ni + i] : 0.0;
-        rr[i] = e.z >= 0 ? r[(size_t)e.z * ni + i] : 0.0;
-    }
-    __syncthreads();
-    const int h = threadIdx.x >> 7;
-    for (int a = threadIdx.x & 127; a < ni; a += 128) {
-        const double sp = e.y >= 0 ? tmv_part(Pj, rl, ni, a, h) : 0.0;
-        const double sq = e.z >= 0 ? tmv_part(Qj, rr, ni, a, h) : 0.0;
-        pp[h][a] = sp + sq;
-    }
-    __syncthreads();
-    for (int a = threadIdx.x; a < ni; a += BCR_ST) r[(size_t)e.x * ni + a] = r[(size_t)e.x * ni + a] - (pp[0][a] + pp[1][a]);
-}
-
-// x_k = A_k^-1 r_k - XB_k x_l - XC_k x_r for the eliminated layers of a level
-// (XB = A_k^-1 B_k, XC = A_k^-1 C_k, formed at factorisation); top: x = A^-1 r
-__global__ void __launch_bounds__(BCR_ST) k_bcr_bwd(int ni, int n, const int4 *__restrict__ el,
-                                                    const int2 *__restrict__ top, const double *__restrict__ Dinv,
-                                                    const double *__restrict__ XB, const double *__restrict__ XC,
-                                                    const double *__restrict__ r, double *__restrict__ x,
-                                                    const vk_colstate *__restrict__ st, double *acc) {
-    const int q = blockIdx.x;
-    if (q >= n) return;
-    int k, left = -1, right = -1, c;
-    if (el) { const int4 e = el[q]; k = e.x; left = e.y; right = e.z; c = e.w; }
-    else { k = top[q].x; c = top[q].y; }
-    if (st && st[c].done) return;
-    const size_t nn = (size_t)ni * ni;
-    __shared__ double rk[VK_NI_MAX], xl[VK_NI_MAX], xr[VK_NI_MAX], pp[2][VK_NI_MAX];
-    for (int i = threadIdx.x; i < ni; i += BCR_ST) {
-        rk[i] = r[(size_t)k * ni + i];
-        xl[i] = left >= 0 ? x[(size_t)left * ni + i] : 0.0;
-        xr[i] = right >= 0 ? x[(size_t)right * ni + i] : 0.0;
-    }
-    __syncthreads();
-    const int h = threadIdx.x >> 7;
-    for (int a = threadIdx.x & 127; a < ni; a += 128) {
-        double v = tmv_part(Dinv + (size_t)k * nn, rk, ni, a, h);
-        if (left >= 0) v = v - tmv_part(XB + (size_t)k * nn, xl, ni, a, h);
-        if (right >= 0) v = v - tmv_part(XC + (size_t)k * nn, xr, ni, a, h);
-        pp[h][a] = v;
-    }
-    __syncthreads();
-    for (int a = threadIdx.x; a < ni; a += BCR_ST) {
-        const double t = pp[0][a] + pp[1][a];
-        x[(size_t)k * ni + a] = t;
-        if (acc) acc[(size_t)k * ni + a] = acc[(size_t)k * ni + a] + t;
-    }
-}
-
-// Solve sweeps for ni <= 128: each block's products are split over row
-// groups of 32 (one workgroup each, grid y), so a block's operators are
-// read by several CUs at once; 256 threads, thread t owns row a0 + t % 32
-// and part h = t / 32 of the b range (chunks of ceil(ni/8) <= 16).  Every
-// operator entry a thread needs is loaded into registers before the first
-// product, and the eight partial sums of a row are combined through LDS in
-// part order.
-constexpr int MV_NT = 256, MV_RG = 32, MV_SP = 8, MV_CH = 16, MV_NIMAX = 128;
-
-__device__ __forceinline__ void mv_load(double (&m)[MV_CH], const double *__restrict__ Mt, int ni, int a, int h,
-                                        int ch) {
+// m[i] = Mt[h ch + i][a], zero past the block (out of the buffer's range)
+template <int CH>
+__device__ __forceinline__ void mv_load(double (&m)[CH], const double *Mt, int ni, int a, int h, int ch) {
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(Mt), (short)0, ni * ni * 8, 0x00020000);
+    const int voff = (h * ch * ni + min(a, ni - 1)) * 8;
 #pragma unroll
-    for (int i = 0; i < MV_CH; i++) {
-        const int b = h * ch + i;
-        m[i] = (i < ch && b < ni && a < ni) ? Mt[(size_t)b * ni + a] : 0.0;
-    }
+    for (int i = 0; i < CH; i++)
+        if (i < ch)
+            m[i] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, voff + i * ni * 8, 0, 0));
 }
 
-__device__ __forceinline__ double mv_dot(const double (&m)[MV_CH], const double *v, int ni, int h, int ch) {
+// v: MV_SP CH entries, zero past the block
+template <int CH>
+__device__ __forceinline__ double mv_dot(const double (&m)[CH], const double *v, int h, int ch) {
     double s0 = 0.0, s1 = 0.0;
 #pragma unroll
-    for (int i = 0; i < MV_CH; i += 2) {
-        const int b = h * ch + i;
-        if (i < ch && b < ni) s0 = fma(m[i], v[b], s0);
-        if (i + 1 < ch && b + 1 < ni) s1 = fma(m[i + 1], v[b + 1], s1);
+    for (int i = 0; i < CH; i += 2) {
+        if (i < ch) s0 = fma(m[i], v[h * ch + i], s0);
+        if (i + 1 < ch) s1 = fma(m[i + 1], v[h * ch + i + 1], s1);
     }
     return s0 + s1;
 }
@@ -365,6 +283,7 @@ __device__ __forceinline__ double mv_dot(const double (&m)[MV_CH], const double 
 // eliminated layers' right-hand sides into r, each layer once: by its
 // right survivor, or by its left one where it ends the column (no layer
 // beyond it: sflag bit 1 clear).
+template <int CH>
 __global__ void __launch_bounds__(MV_NT) k_bcr_fwd_s(int ni, int n, const int4 *__restrict__ sv, int slot0,
                                                      const double *__restrict__ P, const double *__restrict__ Q,
                                                      const double *rin, double *r, const int *__restrict__ sflag,
@@ -375,16 +294,16 @@ __global__ void __launch_bounds__(MV_NT) k_bcr_fwd_s(int ni, int n, const int4 *
     if (st && st[e.w].done) return;
     const size_t nn = (size_t)ni * ni;
     const int lr = threadIdx.x % MV_RG, a = a0 + lr, h = threadIdx.x / MV_RG, ch = (ni + MV_SP - 1) / MV_SP;
-    double mp[MV_CH], mq[MV_CH];
-    mv_load(mp, P + (size_t)(slot0 + q) * nn, e.y >= 0 ? ni : 0, a, h, ch);
-    mv_load(mq, Q + (size_t)(slot0 + q) * nn, e.z >= 0 ? ni : 0, a, h, ch);
-    __shared__ double rl[MV_NIMAX], rr[MV_NIMAX], pp[MV_SP][MV_RG];
-    for (int i = threadIdx.x; i < ni; i += MV_NT) {
-        rl[i] = e.y >= 0 ? rin[(size_t)e.y * ni + i] : 0.0;
-        rr[i] = e.z >= 0 ? rin[(size_t)e.z * ni + i] : 0.0;
+    double mp[CH] = {}, mq[CH] = {};
+    if (e.y >= 0) mv_load<CH>(mp, P + (size_t)(slot0 + q) * nn, ni, a, h, ch);
+    if (e.z >= 0) mv_load<CH>(mq, Q + (size_t)(slot0 + q) * nn, ni, a, h, ch);
+    __shared__ double rl[MV_SP * CH], rr[MV_SP * CH], pp[MV_SP][MV_RG];
+    for (int i = threadIdx.x; i < MV_SP * CH; i += MV_NT) {
+        rl[i] = i < ni && e.y >= 0 ? rin[(size_t)e.y * ni + i] : 0.0;
+        rr[i] = i < ni && e.z >= 0 ? rin[(size_t)e.z * ni + i] : 0.0;
     }
     __syncthreads();
-    pp[h][lr] = mv_dot(mp, rl, ni, h, ch) + mv_dot(mq, rr, ni, h, ch);
+    pp[h][lr] = mv_dot<CH>(mp, rl, h, ch) + mv_dot<CH>(mq, rr, h, ch);
     __syncthreads();
     if (threadIdx.x < MV_RG && a < ni) {
         double t = 0.0;
@@ -398,6 +317,7 @@ __global__ void __launch_bounds__(MV_NT) k_bcr_fwd_s(int ni, int n, const int4 *
     }
 }
 
+template <int CH>
 __global__ void __launch_bounds__(MV_NT) k_bcr_bwd_s(int ni, int n, const int4 *__restrict__ el,
                                                      const int2 *__restrict__ top, const double *__restrict__ Dinv,
                                                      const double *__restrict__ XB, const double *__restrict__ XC,
@@ -412,18 +332,18 @@ __global__ void __launch_bounds__(MV_NT) k_bcr_bwd_s(int ni, int n, const int4 *
     const size_t nn = (size_t)ni * ni;
     const int lr = threadIdx.x % MV_RG, a = a0 + lr, h = threadIdx.x / MV_RG, ch = (ni + MV_SP - 1) / MV_SP;
     // x_k = A_k^-1 r_k - XB x_l - XC x_r: one pass over three operators
-    double mx[MV_CH], mb[MV_CH], mc[MV_CH];
-    mv_load(mx, Dinv + (size_t)k * nn, ni, a, h, ch);   // X[m][a] = inv[a][m]: the transposed inverse
-    mv_load(mb, XB + (size_t)k * nn, left >= 0 ? ni : 0, a, h, ch);
-    mv_load(mc, XC + (size_t)k * nn, right >= 0 ? ni : 0, a, h, ch);
-    __shared__ double rk[MV_NIMAX], xl[MV_NIMAX], xr[MV_NIMAX], pp[MV_SP][MV_RG];
-    for (int i = threadIdx.x; i < ni; i += MV_NT) {
-        rk[i] = r[(size_t)k * ni + i];
-        xl[i] = left >= 0 ? x[(size_t)left * ni + i] : 0.0;
-        xr[i] = right >= 0 ? x[(size_t)right * ni + i] : 0.0;
+    double mx[CH], mb[CH] = {}, mc[CH] = {};
+    mv_load<CH>(mx, Dinv + (size_t)k * nn, ni, a, h, ch);   // X[m][a] = inv[a][m]: the transposed inverse
+    if (left >= 0) mv_load<CH>(mb, XB + (size_t)k * nn, ni, a, h, ch);
+    if (right >= 0) mv_load<CH>(mc, XC + (size_t)k * nn, ni, a, h, ch);
+    __shared__ double rk[MV_SP * CH], xl[MV_SP * CH], xr[MV_SP * CH], pp[MV_SP][MV_RG];
+    for (int i = threadIdx.x; i < MV_SP * CH; i += MV_NT) {
+        rk[i] = i < ni ? r[(size_t)k * ni + i] : 0.0;
+        xl[i] = i < ni && left >= 0 ? x[(size_t)left * ni + i] : 0.0;
+        xr[i] = i < ni && right >= 0 ? x[(size_t)right * ni + i] : 0.0;
     }
     __syncthreads();
-    pp[h][lr] = (mv_dot(mx, rk, ni, h, ch) - mv_dot(mb, xl, ni, h, ch)) - mv_dot(mc, xr, ni, h, ch);
+    pp[h][lr] = (mv_dot<CH>(mx, rk, h, ch) - mv_dot<CH>(mb, xl, h, ch)) - mv_dot<CH>(mc, xr, h, ch);
     __syncthreads();
     if (threadIdx.x < MV_RG && a < ni) {
         double t = 0.0;
@@ -441,7 +361,7 @@ __global__ void __launch_bounds__(MV_NT) k_bcr_bwd_s(int ni, int n, const int4 *
 // in k_bcr_fwd_s / k_bcr_bwd_s (same partition of the columns, same order
 // of the sums; their product with an absent neighbour is exactly +0.0 and
 // stands here as that constant), so the results are theirs.
-constexpr int TAIL_G = 3, TAIL_NIMAX = TAIL_G * MV_RG;
+constexpr int TAIL_G = 3, TAIL_NIMAX = TAIL_G * MV_RG, TAIL_CH = TAIL_NIMAX / MV_SP;
 __global__ void __launch_bounds__(MV_NT *TAIL_G) k_bcr_tail_s(int ni, const int4 *__restrict__ sv, int slot0,
                                                               const int4 *__restrict__ el, const double *__restrict__ Q,
                                                               const double *__restrict__ Dinv,
@@ -454,13 +374,17 @@ __global__ void __launch_bounds__(MV_NT *TAIL_G) k_bcr_tail_s(int ni, const int4
     const int lr = tt % MV_RG, a = MV_RG * g + lr, h = tt / MV_RG, ch = (ni + MV_SP - 1) / MV_SP;
     const int ks = es.x, ke = ee.x;
     // every operator up front: Q_s, A_s^-1, A_e^-1, XB_e
-    double mq[MV_CH], mxs[MV_CH], mxe[MV_CH], mb[MV_CH];
-    mv_load(mq, Q + (size_t)slot0 * nn, ni, a, h, ch);
-    mv_load(mxs, Dinv + (size_t)ks * nn, ni, a, h, ch);
-    mv_load(mxe, Dinv + (size_t)ke * nn, ni, a, h, ch);
-    mv_load(mb, XB + (size_t)ke * nn, ni, a, h, ch);
+    constexpr int CH = TAIL_CH;
+    double mq[CH], mxs[CH], mxe[CH], mb[CH];
+    mv_load<CH>(mq, Q + (size_t)slot0 * nn, ni, a, h, ch);
+    mv_load<CH>(mxs, Dinv + (size_t)ks * nn, ni, a, h, ch);
+    mv_load<CH>(mxe, Dinv + (size_t)ke * nn, ni, a, h, ch);
+    mv_load<CH>(mb, XB + (size_t)ke * nn, ni, a, h, ch);
     __shared__ double re[TAIL_NIMAX], rs[TAIL_NIMAX], xs[TAIL_NIMAX], pp[TAIL_G][MV_SP][MV_RG];
-    for (int i = threadIdx.x; i < ni; i += blockDim.x) re[i] = r[(size_t)ke * ni + i];
+    for (int i = threadIdx.x; i < TAIL_NIMAX; i += blockDim.x) {
+        re[i] = i < ni ? r[(size_t)ke * ni + i] : 0.0;
+        rs[i] = xs[i] = 0.0;                     // past the block; the block's entries follow below
+    }
     __syncthreads();
     auto total = [&]() {
         double t = 0.0;
@@ -469,7 +393,7 @@ __global__ void __launch_bounds__(MV_NT *TAIL_G) k_bcr_tail_s(int ni, const int4
         return t;
     };
     // forward: r_s -= P_s r_l + Q_s r_r, no left neighbour
-    pp[g][h][lr] = 0.0 + mv_dot(mq, re, ni, h, ch);
+    pp[g][h][lr] = 0.0 + mv_dot<CH>(mq, re, h, ch);
     __syncthreads();
     if (h == 0 && a < ni) {
         const double v = r[(size_t)ks * ni + a] - total();
@@ -478,7 +402,7 @@ __global__ void __launch_bounds__(MV_NT *TAIL_G) k_bcr_tail_s(int ni, const int4
     }
     __syncthreads();
     // top: x_s = A_s^-1 r_s, no neighbours
-    pp[g][h][lr] = (mv_dot(mxs, rs, ni, h, ch) - 0.0) - 0.0;
+    pp[g][h][lr] = (mv_dot<CH>(mxs, rs, h, ch) - 0.0) - 0.0;
     __syncthreads();
     if (h == 0 && a < ni) {
         const double t = total();
@@ -488,7 +412,7 @@ __global__ void __launch_bounds__(MV_NT *TAIL_G) k_bcr_tail_s(int ni, const int4
     }
     __syncthreads();
     // back-substitution of e: x_e = A_e^-1 r_e - XB_e x_s, no right neighbour
-    pp[g][h][lr] = (mv_dot(mxe, re, ni, h, ch) - mv_dot(mb, xs, ni, h, ch)) - 0.0;
+    pp[g][h][lr] = (mv_dot<CH>(mxe, re, h, ch) - mv_dot<CH>(mb, xs, h, ch)) - 0.0;
     __syncthreads();
     if (h == 0 && a < ni) {
         const double t = total();
@@ -563,45 +487,46 @@ int vk_launch_bcr_factor(int nb, int ni, const vk_columns *cols, const double *D
     }
 }
 
-int vk_launch_bcr_solve(int ni, const vk_columns *cols, const double *Dinv, const double *Lsub, const double *Usup,
-                        const double *in, double *out, double *tmp, const vk_colstate *st, const vk_bcr_ws *ws,
-                        double *acc, hipStream_t s) {
+template <int CH>
+static int launch_bcr_solve(int ni, const vk_columns *cols, const double *Dinv, const double *in, double *out,
+                            double *tmp, const vk_colstate *st, const vk_bcr_ws *ws, double *acc, hipStream_t s) {
     const vk_bcr_sched &b = cols->bcr;
-    const long n = (long)cols->L * ni;
-    // ni <= 128: the row-group sweeps (several workgroups per block); their
-    // level 0 reads `in` and fills tmp itself, the generic sweeps start
-    // from a copy
-    const bool small = ni <= MV_NIMAX;
-    auto bwd = small ? k_bcr_bwd_s : k_bcr_bwd;
-    const int bt = small ? MV_NT : BCR_ST, gy = small ? (ni + MV_RG - 1) / MV_RG : 1;
-    if (!small) hipLaunchKernelGGL(k_copy_d, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, in, tmp);
+    const int gy = (ni + MV_RG - 1) / MV_RG;
     // the last level and the top in one launch (one column, ni <= 96)
-    const bool tail = small && b.tail && ni <= TAIL_NIMAX;
+    const bool tail = b.tail && ni <= TAIL_NIMAX;
+    // level 0 reads `in` and fills tmp
     for (int lev = 0; lev < b.nlev; lev++) {
         const int s0 = b.surv_off[lev], ns = b.surv_off[lev + 1] - s0;
         if (ns <= 0) continue;
         if (tail && lev == b.nlev - 1) {
             const int e0 = b.elim_off[lev];
-            hipLaunchKernelGGL(k_bcr_tail_s, dim3(1), dim3(MV_NT * ((ni + MV_RG - 1) / MV_RG)), 0, s, ni,
-                               b.d_surv + s0, s0, b.d_elim + e0, ws->Q, Dinv, ws->XB, tmp, out, st, acc);
+            hipLaunchKernelGGL(k_bcr_tail_s, dim3(1), dim3(MV_NT * gy), 0, s, ni, b.d_surv + s0, s0, b.d_elim + e0,
+                               ws->Q, Dinv, ws->XB, tmp, out, st, acc);
             break;
         }
-        if (small)
-            hipLaunchKernelGGL(k_bcr_fwd_s, dim3(ns, gy), dim3(bt), 0, s, ni, ns, b.d_surv + s0, s0, ws->P, ws->Q,
-                               lev == 0 ? in : tmp, tmp, lev == 0 ? b.d_sflag + s0 : (const int *)nullptr, st);
-        else
-            hipLaunchKernelGGL(k_bcr_fwd, dim3(ns, gy), dim3(bt), 0, s, ni, ns, b.d_surv + s0, s0, ws->P, ws->Q, tmp,
-                               st);
+        hipLaunchKernelGGL(k_bcr_fwd_s<CH>, dim3(ns, gy), dim3(MV_NT), 0, s, ni, ns, b.d_surv + s0, s0, ws->P, ws->Q,
+                           lev == 0 ? in : tmp, tmp, lev == 0 ? b.d_sflag + s0 : (const int *)nullptr, st);
     }
     if (!tail)
-        hipLaunchKernelGGL(bwd, dim3(b.ntop, gy), dim3(bt), 0, s, ni, b.ntop, (const int4 *)nullptr, b.d_top, Dinv,
-                           ws->XB, ws->XC, tmp, out, st, acc);
+        hipLaunchKernelGGL(k_bcr_bwd_s<CH>, dim3(b.ntop, gy), dim3(MV_NT), 0, s, ni, b.ntop, (const int4 *)nullptr,
+                           b.d_top, Dinv, ws->XB, ws->XC, tmp, out, st, acc);
     for (int lev = b.nlev - 1 - (tail ? 1 : 0); lev >= 0; lev--) {
         const int e0 = b.elim_off[lev], ne = b.elim_off[lev + 1] - e0;
         if (ne > 0)
-            hipLaunchKernelGGL(bwd, dim3(ne, gy), dim3(bt), 0, s, ni, ne, b.d_elim + e0, (const int2 *)nullptr, Dinv,
-                               ws->XB, ws->XC, tmp, out, st, acc);
+            hipLaunchKernelGGL(k_bcr_bwd_s<CH>, dim3(ne, gy), dim3(MV_NT), 0, s, ni, ne, b.d_elim + e0,
+                               (const int2 *)nullptr, Dinv, ws->XB, ws->XC, tmp, out, st, acc);
     }
     VK_CHECK(hipGetLastError());
     return 0;
+}
+
+int vk_launch_bcr_solve(int ni, const vk_columns *cols, const double *Dinv, const double *Lsub, const double *Usup,
+                        const double *in, double *out, double *tmp, const vk_colstate *st, const vk_bcr_ws *ws,
+                        double *acc, hipStream_t s) {
+    // CH: entries of a row a thread holds, MV_SP CH >= ni
+    static_assert(VK_NI_MAX <= MV_SP * 20, "row chunks of the solve sweeps");
+    if (ni <= MV_SP * 8) return launch_bcr_solve<8>(ni, cols, Dinv, in, out, tmp, st, ws, acc, s);
+    if (ni <= MV_SP * 12) return launch_bcr_solve<12>(ni, cols, Dinv, in, out, tmp, st, ws, acc, s);
+    if (ni <= MV_SP * 16) return launch_bcr_solve<16>(ni, cols, Dinv, in, out, tmp, st, ws, acc, s);
+    return launch_bcr_solve<20>(ni, cols, Dinv, in, out, tmp, st, ws, acc, s);
 }
