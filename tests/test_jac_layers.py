@@ -1,4 +1,4 @@
-"""Jacobian and left-hand-side blocks with two layers per workgroup (many
+"""Right-hand sides, Jacobian and left-hand-side blocks with two layers per workgroup (many
 layers) against one (few layers), bit for bit: an odd number of layers, columns
 of different lengths and time steps whose ends fall inside a pair of layers,
 and pairs of reactions with a species twice on one side, in either order, and
@@ -56,7 +56,12 @@ def test_two_layers_per_workgroup(which, nz):
                               stream_handle()), 'vk_jac')
         _lib.check(lib.vk_lhs(b.plan.handle, b.layout.handle, C.byref(b.atm), dptr(b.y), dptr(b.k), mol, dptr(d),
                               dptr(D), dptr(Ls), dptr(Us), stream_handle()), 'vk_lhs')
-        out = [t.cpu().numpy() for t in (J, D, Ls, Us, b.k)]
+        f, g = torch.empty_like(b.y), torch.empty_like(b.y)
+        _lib.check(lib.vk_chemdf(b.plan.handle, b.layout.handle, dptr(b.y), dptr(b.M), dptr(b.k), dptr(f),
+                                 stream_handle()), 'vk_chemdf')
+        _lib.check(lib.vk_diffdf(b.plan.handle, b.layout.handle, C.byref(b.atm), dptr(b.y), mol, dptr(g),
+                                 stream_handle()), 'vk_diffdf')
+        out = [t.cpu().numpy() for t in (J, D, Ls, Us, f, g, b.k)]
         b.close()
         return out
 
@@ -68,10 +73,10 @@ def test_two_layers_per_workgroup(which, nz):
         for i in (0, 1, len(cases) // 2, len(cases) - 1):
             few = blocks(everything[i:i + 1], mol)
             s = slice(off[i], off[i + 1])
-            for a, b in zip(many[:4], few[:4]):
+            for a, b in zip(many[:6], few[:6]):
                 assert np.array_equal(a[s], b)
         col = cases[-1].col
-        J = O.jac_blocks(net, y0[-1], col.M, few[4])
+        J = O.jac_blocks(net, y0[-1], col.M, few[6])
         assert np.array_equal(few[0], J)
         for a, b in zip(few[1:4], O.lhs_blocks(col, y0[-1], dt[-1], J, bool(mol))):
             assert np.array_equal(a, b)

@@ -273,26 +273,6 @@ __device__ inline LayerCtx layer_ctx(const int *off, const int *layer_col, int l
     return x;
 }
 
-// v_p = k_f * prod(reac) - k_r * prod(prod), left to right (make_chem_funs.py:293-315);
-// the four terms of a side are one 16-byte load
-__device__ inline double side_product(int4 t4, double kcol, const double *yl, double m, int ni) {
-    const int t[4] = {t4.x, t4.y, t4.z, t4.w};
-    double a = kcol;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        if (t[q] == -2) continue;
-        a = a * (t[q] == -1 ? m : yl[VK_IX(t[q], ni, VK_SITE_SPECIES)]);
-    }
-    return a;
-}
-
-__device__ inline double pair_rate(const int4 *reac, const int4 *prod, const double *kl, const double *yl,
-                                   double m, int p, int ni) {
-    const double a = side_product(reac[p], kl[2 * p], yl, m, ni);
-    const double b = side_product(prod[p], kl[2 * p + 1], yl, m, ni);
-    return a - b;
-}
-
 // d/dy_sp of kcol * prod(terms), yl[LG s] the amount of species s
 template <int LG>
 __device__ inline double dside(int4 t4, double kcol, const double *yl, double m, int sp, int ni) {
@@ -329,69 +309,110 @@ __device__ inline void ysum_around(const double *ysum, const LayerCtx &x, double
 }
 
 // ---------------------------------------------------------------------------
-// chemdf + diffdf (+ stage-2 term), one workgroup per layer
+// chemdf + diffdf (+ stage-2 term), one workgroup per LG layers
 // mode bit 0: include chemistry, bit 1: include diffusion
+//
+// Bound by the table reads: a pair is eight bytes (its amounts' indices), the
+// species' terms lie term by term over the species, so that the lanes of a
+// wave read neighbouring ones, and with two layers a workgroup reads a pair
+// once for both.  36 000 layers of 93 species, 620 pairs: 320 -> 263 us; 150
+// layers: 13.5 -> 12.4 us.
 // ---------------------------------------------------------------------------
 
+template <int LG>
 __global__ void __launch_bounds__(BLK) k_rhs(
-    int ni, int npairs, int nchem, const int *__restrict__ off, const int *__restrict__ layer_col,
-    const int *__restrict__ reac, const int *__restrict__ prod, const int *__restrict__ chem_ptr,
-    const int2 *__restrict__ chem_ent, const double *__restrict__ ms,
-    const double *__restrict__ alpha, vk_atm atm, const double *__restrict__ y, const double *__restrict__ k,
-    const double *__restrict__ M, int mode, int mol, const double *__restrict__ k1,
+    int L, int ni, int npairs, int nchem, const int *__restrict__ off, const int *__restrict__ layer_col,
+    const uint2 *__restrict__ pair_tab, const int *__restrict__ chem_ptr, const int2 *__restrict__ chem_ent,
+    const double *__restrict__ ms, const double *__restrict__ alpha, vk_atm atm, const double *__restrict__ y,
+    const double *__restrict__ k, const double *__restrict__ M, int mode, int mol, const double *__restrict__ k1,
     const double *__restrict__ dtc, const double *__restrict__ ysum, const vk_colstate *__restrict__ st,
     double *__restrict__ out) {
-    extern __shared__ double smem[];
-    double *yl = smem;              // ni
-    double *v = smem + VK_NI_MAX;   // npairs
-    const int l = blockIdx.x;
-    LayerCtx x = layer_ctx(off, layer_col, l);
-    if (st && st[x.c].done) return;
-    const double *yrow = y + (size_t)l * ni;
-    for (int i = threadIdx.x; i < ni; i += blockDim.x) yl[i] = yrow[i];
-    double ysm = 0.0, ys0 = 0.0, ysp = 0.0;
-    if (mode & 2) ysum_around(ysum, x, ysm, ys0, ysp);
+    extern __shared__ __align__(16) double smem[];
+    double *v = smem;                  // npairs x LG: rates of the pairs
+    double *yl = smem + LG * npairs;   // (ni + 2) x LG: amounts, then M and one
+    const int l0 = blockIdx.x * LG;
+    LayerCtx xs[LG];
+    bool on[LG], any = false;
+#pragma unroll
+    for (int a = 0; a < LG; a++) {
+        xs[a] = layer_ctx(off, layer_col, min(l0 + a, L - 1));
+        on[a] = l0 + a < L && !(st && st[xs[a].c].done);
+        any = any || on[a];
+    }
+    if (!any) return;
+    for (int q = threadIdx.x; q < ni + 2; q += BLK)
+#pragma unroll
+        for (int a = 0; a < LG; a++)
+            yl[LG * q + a] = q < ni ? y[(size_t)xs[a].l * ni + q] : (q > ni ? 1.0 : (mode & 1 ? M[xs[a].l] : 0.0));
     __syncthreads();
     if (mode & 1) {
-        const double *kl = k + (size_t)l * 2 * npairs;
-        double m = M[l];
-        for (int p = threadIdx.x; p < npairs; p += blockDim.x)
-            v[p] = pair_rate((const int4 *)reac, (const int4 *)prod, kl, yl, m, p, ni);
+        // v_p = k_f * prod(reac) - k_r * prod(prod), left to right (make_chem_funs.py:293-315)
+        for (int p = threadIdx.x; p < npairs; p += BLK) {
+            const uint2 t = pair_tab[p];
+            double f[LG], r[LG];
+#pragma unroll
+            for (int a = 0; a < LG; a++) {
+                const double *kl = k + ((size_t)xs[a].l * npairs + p) * 2;
+                f[a] = kl[0];
+                r[a] = kl[1];
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const double *yf = yl + LG * VK_IX(t.x >> 8 * q & 255, ni + 2, VK_SITE_SPECIES);
+                const double *yr = yl + LG * VK_IX(t.y >> 8 * q & 255, ni + 2, VK_SITE_SPECIES);
+#pragma unroll
+                for (int a = 0; a < LG; a++) {
+                    f[a] = f[a] * yf[a];
+                    r[a] = r[a] * yr[a];
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < LG; a++) v[LG * p + a] = f[a] - r[a];
+        }
         __syncthreads();
     }
-    ColAtm ca = col_atm(atm, x.c, x.off, x.nz, ni);
-    double c2 = 0.0;
-    if (k1) c2 = 2. / (R_ROS * dtc[x.c]);
-    for (int i = threadIdx.x; i < ni; i += blockDim.x) {
+    for (int q = threadIdx.x; q < LG * ni; q += BLK) {
+        const int a = q / ni, i = q - a * ni;
+        LayerCtx x = xs[0];
+        bool go = on[0];
+        if (LG > 1 && a > 0) {
+            x = xs[LG - 1];
+            go = on[LG - 1];
+        }
+        if (!go) continue;
+        const int l = x.l;
+        double ysm = 0.0, ys0 = 0.0, ysp = 0.0;
+        if (mode & 2) ysum_around(ysum, x, ysm, ys0, ysp);
         double chem = 0.0;
         if (mode & 1) {
-            const int lo = chem_ptr[i], hi = chem_ptr[i + 1];
-            if (lo < hi) {
-                int2 t = chem_ent[VK_IX(lo, nchem, VK_SITE_CHEM)];   // (pair, sign)
-                chem = t.y * v[VK_IX(t.x, npairs, VK_SITE_PAIR)];
+            const int n = chem_ptr[i + 1] - chem_ptr[i];
+            if (n > 0) {
+                int2 t = chem_ent[VK_IX(i, nchem, VK_SITE_CHEM)];   // (pair, sign)
+                chem = t.y * v[LG * VK_IX(t.x, npairs, VK_SITE_PAIR) + a];
                 // the terms in order, eight entries loaded ahead of their sums
-                int e = lo + 1;
-                for (; e + 8 <= hi; e += 8) {
+                int e = 1;
+                for (; e + 8 <= n; e += 8) {
                     int2 tt[8];
 #pragma unroll
-                    for (int u = 0; u < 8; u++) tt[u] = chem_ent[VK_IX(e + u, nchem, VK_SITE_CHEM)];
+                    for (int u = 0; u < 8; u++) tt[u] = chem_ent[VK_IX((e + u) * ni + i, nchem, VK_SITE_CHEM)];
 #pragma unroll
-                    for (int u = 0; u < 8; u++) chem = chem + tt[u].y * v[VK_IX(tt[u].x, npairs, VK_SITE_PAIR)];
+                    for (int u = 0; u < 8; u++) chem = chem + tt[u].y * v[LG * VK_IX(tt[u].x, npairs, VK_SITE_PAIR) + a];
                 }
-                for (; e < hi; e++) {
-                    t = chem_ent[VK_IX(e, nchem, VK_SITE_CHEM)];
-                    chem = chem + t.y * v[VK_IX(t.x, npairs, VK_SITE_PAIR)];
+                for (; e < n; e++) {
+                    t = chem_ent[VK_IX(e * ni + i, nchem, VK_SITE_CHEM)];
+                    chem = chem + t.y * v[LG * VK_IX(t.x, npairs, VK_SITE_PAIR) + a];
                 }
             }
         }
+        const ColAtm ca = col_atm(atm, x.c, x.off, x.nz, ni);
         double val = chem;
         if (mode & 2) {
             double ym = x.j > 0 ? y[(size_t)(l - 1) * ni + i] : 0.0;
             double yp = x.j < x.nz - 1 ? y[(size_t)(l + 1) * ni + i] : 0.0;
-            double d = diff_value(ca, x.j, i, ysm, ys0, ysp, ym, yl[i], yp, ms[i], alpha[i], mol != 0);
+            double d = diff_value(ca, x.j, i, ysm, ys0, ysp, ym, yl[LG * i + a], yp, ms[i], alpha[i], mol != 0);
             val = (mode & 1) ? chem + d : d;
         }
-        if (k1) val = val - c2 * k1[(size_t)l * ni + i];
+        if (k1) val = val - 2. / (R_ROS * dtc[x.c]) * k1[(size_t)l * ni + i];
         out[(size_t)l * ni + i] = val;
     }
 }
@@ -608,7 +629,9 @@ __global__ void __launch_bounds__(BLK *LG, 4) k_jac_lhs(
 
 static inline hipStream_t S(void *s) { return (hipStream_t)s; }
 
-static size_t rhs_smem(const vk_plan *p) { return sizeof(double) * (VK_NI_MAX + (size_t)p->npairs); }
+static size_t rhs_smem(const vk_plan *p, int layers) {
+    return sizeof(double) * layers * (p->ni + 2 + (size_t)p->npairs);
+}
 static size_t jac_smem(const vk_plan *p, int layers) {
     return sizeof(double) * layers * (4 * VK_NI_MAX + 2 + (size_t)p->nslot);
 }
@@ -645,10 +668,17 @@ int vk_launch_rhs(const vk_plan *plan, const vk_columns *cols, const vk_atm *atm
         int r = launch_ysum(cols, plan->ni, y, ysum, s);
         if (r) return r;
     }
-    hipLaunchKernelGGL(k_rhs, dim3(cols->L), dim3(BLK), rhs_smem(plan), s, plan->ni, plan->npairs, plan->nchem,
-                       cols->d_off,
-                       cols->d_layer_col, plan->reac, plan->prod, plan->chem_ptr, plan->chem_ent, plan->ms,
-                       plan->alpha, a, y, k, atm->M, mode, mol, k1, dtc, ysum, st, out);
+    auto launch = [&](auto kernel, int layers) {
+        hipLaunchKernelGGL(kernel, dim3((cols->L + layers - 1) / layers), dim3(BLK), rhs_smem(plan, layers), s, cols->L,
+                           plan->ni, plan->npairs, plan->nchem_ent, cols->d_off, cols->d_layer_col, plan->pair_tab,
+                           plan->chem_ptr, plan->chem_ent, plan->ms, plan->alpha, a, y, k, atm->M, mode, mol, k1, dtc,
+                           ysum, st, out);
+    };
+    // two layers a workgroup where a CU holds eight such workgroups and still gets several
+    if (rhs_smem(plan, 2) <= 20 * 1024 && cols->L >= 12 * vk_device_cus())
+        launch(k_rhs<2>, 2);
+    else
+        launch(k_rhs<1>, 1);
     VK_CHECK(hipGetLastError());
     return 0;
 }

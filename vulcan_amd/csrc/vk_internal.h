@@ -66,7 +66,9 @@ struct vk_plan {
     int *reac, *prod, *kind, *rev;
     double *par, *nasa9, *atom_mat, *ms, *alpha;
     int *chem_ptr, *chem_pair, *chem_sign;
-    int2 *chem_ent;            // (chem_pair, chem_sign) interleaved
+    int nchem_ent;             // entries of chem_ent
+    int2 *chem_ent;            // (pair, sign) of species i's e-th term at e ni + i (chem_ptr gives how many)
+    uint2 *pair_tab;           // the amounts of a pair's reactants and products, a byte each: species; ni: M; ni + 1: one
     int *jac_map, *jac_ptr, *jac_slot;
     int njent;                 // entries with chemical terms plus the diagonal
     int4 *jac_ent;             // (dense index, first term, end of terms, row), longest term lists first

@@ -542,9 +542,25 @@ extern "C" int vk_plan_create(const vk_network_desc *n, vk_plan **out) {
         light.assign(ent.begin() + p->njheavy, ent.end());
     }
     if (!r) {
-        std::vector<int2> ce((size_t)n->nchem);
-        for (size_t q = 0; q < ce.size(); q++) ce[q] = make_int2(n->chem_pair[q], n->chem_sign[q]);
+        int most = 1;
+        for (int i = 0; i < n->ni; i++) most = std::max(most, n->chem_ptr[i + 1] - n->chem_ptr[i]);
+        std::vector<int2> ce((size_t)most * n->ni, make_int2(0, 0));
+        for (int i = 0; i < n->ni; i++)
+            for (int e = n->chem_ptr[i]; e < n->chem_ptr[i + 1]; e++)
+                ce[(size_t)(e - n->chem_ptr[i]) * n->ni + i] = make_int2(n->chem_pair[e], n->chem_sign[e]);
+        p->nchem_ent = (int)ce.size();
         r = upload(v, &p->chem_ent, ce.data(), ce.size());
+        std::vector<uint2> pt((size_t)n->npairs);
+        auto bytes = [&](const int *t) {
+            unsigned w = 0;
+            for (int q = 0; q < 4; q++) {
+                const int f = t[q] == -2 ? n->ni + 1 : (t[q] == -1 ? n->ni : t[q]);
+                w |= (unsigned)(f < 0 || f > n->ni + 1 ? 255 : f) << 8 * q;
+            }
+            return w;
+        };
+        for (int q = 0; q < n->npairs; q++) pt[q] = make_uint2(bytes(n->reac + 4 * q), bytes(n->prod + 4 * q));
+        r = r ? r : upload(v, &p->pair_tab, pt.data(), pt.size());
     }
     if (!r) {
         std::vector<int> terms((size_t)n->njac);
