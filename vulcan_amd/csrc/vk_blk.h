@@ -46,6 +46,15 @@ struct BlkGrid {
 // ---------------------------------------------------------------------------
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
+// Pivots per panel of blk_invert_diag.  A pivot step broadcasts a row of the
+// panel and updates its columns, so narrow panels halve it, and twice as many
+// panels cost a round of publishing and two barriers each: measured 8 against
+// 16 with 48 species (80 columns' chains) 0.89 against 1.03 ms, 93 species one
+// block 38 against 31 us and 256 columns' chains 3.68 against 3.65 ms, 150
+// species one block 113 against 121 us and 80 columns' chains 7.4 against 7.6 ms.
+template <int NB>
+constexpr int DIAG_PW = NB <= 3 || blk_nt(NB) > NT ? 8 : 16;
+
 template <int NB>
 struct BlkShared {
     static constexpr int N16 = 16 * NB;
@@ -65,9 +74,9 @@ struct BlkShared {
             double park[PARK ? 4 * ((NB + 1) / 2) * ((NB + 3) / 4) : 1][64];
         };
         struct {                      // blk_invert_diag
-            double dpan[16][N16 + 1];     // panel columns, [k][row]
-            double dfac[16][N16 + 1];     // the factored panel
-            double drb[2][16][N16];       // old pivot rows, [s][col], by panel parity
+            double dpan[DIAG_PW<NB>][N16 + 1];   // panel columns, [k][row]
+            double dfac[DIAG_PW<NB>][N16 + 1];   // the factored panel
+            double drb[2][DIAG_PW<NB>][N16];     // old pivot rows, [s][col], by panel parity
             double diag[N16];             // the block's diagonal as given
         };
     };
@@ -325,7 +334,7 @@ __device__ __forceinline__ void blk_invert(f64x4 (&acc)[BlkGrid<NB>::TBR][BlkGri
 // wave-wide maximum, a row hand-over through LDS and the whole panel's
 // update per step, some 900 cycles (36 of an inversion's 58 us at 93 rows)
 // while the workgroup's other waves wait.  With the pivot rows known in
-// advance, every wave holds the panel's 16 pivot rows in its lanes 0..15
+// advance, every wave holds the panel's pivot rows in its first lanes
 // (all waves run the same steps on them) and its own share of the other rows
 // in the lanes above, one row a lane: the pivot row of a step is lane kk's,
 // read by v_readlane into scalar registers, no row crosses waves, and a
@@ -348,7 +357,8 @@ __device__ __forceinline__ void blk_invert(f64x4 (&acc)[BlkGrid<NB>::TBR][BlkGri
 //
 // One column of 150 layers and 93 species: factorisation and two solves 0.77
 // -> 0.54 ms; chains of one column 5.25 -> 3.08 ms, of 256 columns (80 to 200
-// layers) 9.3 -> 6.5 ms; nine 150-species columns 17.9 -> 12.5 ms.
+// layers) 9.3 -> 6.5 ms (5.6 with the chains' own Schur term and sweeps); nine
+// 150-species columns 17.9 -> 12.5 ms.
 // Returns whether the inverse has been written (uniform over the workgroup).
 // ---------------------------------------------------------------------------
 constexpr double DIAG_KEEP = 0.5;
@@ -365,16 +375,16 @@ __device__ __forceinline__ bool blk_invert_diag(f64x4 (&acc)[BlkGrid<NB>::TBR][B
                                                 double *__restrict__ X, BlkShared<NB> &sh) {
     using G = BlkGrid<NB>;
     constexpr int N16 = 16 * NB, TBR = G::TBR, TBC = G::TBC, WC = G::WC;
-    constexpr int SHARE = (N16 - 16 + G::NW - 1) / G::NW;   // rows outside the pivot tile, per wave
-    static_assert(SHARE <= 48, "a wave's lanes hold the pivot rows and its share");
+    constexpr int PW = DIAG_PW<NB>, SHARE = (N16 - PW + G::NW - 1) / G::NW;   // rows outside the pivots', per wave
+    static_assert(SHARE + PW <= 64 && 16 % PW == 0 && PW % 4 == 0, "a wave's lanes hold the pivot rows and its share");
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));   // as in blk_load_schur: no index of this function lives across the caller's loop
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;   // uniform: the tile tests are scalar branches
     const int wr = w / WC, wc = w % WC;
     const int lg = l >> 4, lc = l & 15;
-    const int npan = (ni + 15) >> 4;
+    const int npan = (ni + PW - 1) / PW;
     // the padding is the identity's: its pivots are 1 and touch nothing, so
-    // that every panel runs its 16 steps without a test
+    // that every panel runs all its steps without a test
 #pragma unroll
     for (int ti = 0; ti < TBR; ti++)
 #pragma unroll
@@ -391,10 +401,12 @@ __device__ __forceinline__ bool blk_invert_diag(f64x4 (&acc)[BlkGrid<NB>::TBR][B
     if (tid == 0) sh.refused = 0;
     for (int pb = 0; pb < npan; pb++) {
         double(*rb)[N16] = sh.drb[pb & 1];
-        const int p0 = 16 * pb;
-        // the owners of column block and row block pb publish them and clear
-        // their tiles: the update below then writes them like any other (the
-        // panel's tiles as the factored panel times the identity)
+        // the panel lies in tile row and column tb, at so
+        const int p0 = PW * pb, tb = p0 >> 4, so = p0 & 15;
+        const bool pc = lc - so >= 0 && lc - so < PW;      // the lane's column of tile tb is in the panel
+        // the owners of the panel's columns and rows publish them and clear
+        // them: the update below then writes them like any other entry (the
+        // panel's columns as the factored panel times the identity)
 #pragma unroll
         for (int ti = 0; ti < TBR; ti++) {
             const int bi = wr + 2 * ti;
@@ -403,74 +415,80 @@ __device__ __forceinline__ bool blk_invert_diag(f64x4 (&acc)[BlkGrid<NB>::TBR][B
             for (int tj = 0; tj < TBC; tj++) {
                 const int bj = wc + WC * tj;
                 if (bj >= NB) continue;
-                if (bj == pb) {
+                if (bj == tb) {
 #pragma unroll
-                    for (int r = 0; r < 4; r++) sh.dpan[lc][16 * bi + 4 * r + lg] = acc[ti][tj][r];
-                    acc[ti][tj] = f64x4{0.0, 0.0, 0.0, 0.0};
-                } else if (bi == pb) {
+                    for (int r = 0; r < 4; r++) {
+                        if (pc) sh.dpan[lc - so][16 * bi + 4 * r + lg] = acc[ti][tj][r];
+                        acc[ti][tj][r] = pc ? 0.0 : acc[ti][tj][r];
+                    }
+                }
+                if (bi == tb) {
 #pragma unroll
-                    for (int r = 0; r < 4; r++) rb[4 * r + lg][16 * bj + lc] = acc[ti][tj][r];
-                    acc[ti][tj] = f64x4{0.0, 0.0, 0.0, 0.0};
+                    for (int r = 0; r < 4; r++) {
+                        const int k = 4 * r - so;            // uniform: four pivot rows or none
+                        if (k >= 0 && k < PW) {
+                            const double one = lc - so == k + lg ? 1.0 : 0.0;
+                            rb[k + lg][16 * bj + lc] = bj == tb && pc ? one : acc[ti][tj][r];
+                            acc[ti][tj][r] = 0.0;
+                        }
+                    }
                 }
             }
         }
         __syncthreads();
         {
             // lane -> row: the pivot rows, then this wave's share of the others
-            const int o = w * SHARE + l - 16;
-            const bool other = l >= 16 && l < 16 + SHARE && o < N16 - 16;
-            const int row = l < 16 ? p0 + l : (other ? (o < p0 ? o : o + 16) : p0);
-            double v[16], pinv = 1.0;
+            const int o = w * SHARE + l - PW;
+            const bool other = l >= PW && l < PW + SHARE && o < N16 - PW;
+            const int row = l < PW ? p0 + l : (other ? (o < p0 ? o : o + PW) : p0);
+            double v[PW], pinv = 1.0;
 #pragma unroll
-            for (int k = 0; k < 16; k++) v[k] = sh.dpan[k][row];
+            for (int k = 0; k < PW; k++) v[k] = sh.dpan[k][row];
 #pragma unroll
-            for (int kk = 0; kk < 16; kk++) {
+            for (int kk = 0; kk < PW; kk++) {
                 const bool own = l == kk;
                 // the pivot row, every entry into scalar registers of its own
                 // (a shared pair would serialise read and use)
-                double p[16];
+                double p[PW];
 #pragma unroll
-                for (int k = 0; k < 16; k++) p[k] = lane_bcast(v[k], kk);
+                for (int k = 0; k < PW; k++) p[k] = lane_bcast(v[k], kk);
                 const double inv = blk_recip(p[kk]);
                 const double f = own ? 0.0 : v[kk] * inv;
 #pragma unroll
-                for (int k = 0; k < 16; k++) asm volatile("" : "+s"(p[k]));
+                for (int k = 0; k < PW; k++) asm volatile("" : "+s"(p[k]));
 #pragma unroll
-                for (int j = 1; j < 16; j++) {
-                    const int k = (kk + j) & 15;      // the next pivot's column first
+                for (int j = 1; j < PW; j++) {
+                    const int k = (kk + j) % PW;      // the next pivot's column first
                     v[k] = fma(-f, p[k], v[k]);
                 }
                 v[kk] = own ? 1.0 : -f;
                 pinv = own ? inv : pinv;
             }
-            if (w == 0 && l < 16 && !(sh.diag[row] * pinv >= DIAG_KEEP)) sh.refused = 1;
-            if (other || (l < 16 && w == 0)) {
+            if (w == 0 && l < PW && !(sh.diag[row] * pinv >= DIAG_KEEP)) sh.refused = 1;
+            if (other || (l < PW && w == 0)) {
 #pragma unroll
-                for (int k = 0; k < 16; k++) sh.dfac[k][row] = v[k] * pinv;
+                for (int k = 0; k < PW; k++) sh.dfac[k][row] = v[k] * pinv;
             }
         }
         __syncthreads();
         if (__builtin_amdgcn_readfirstlane(sh.refused)) return false;
-        // rank-16 update on MFMA (tiles past the block read block 0's
+        // rank-PW update on MFMA (tiles past the block read block 0's
         // operands, their values are never used)
-        double b[TBC][4];
+        double b[TBC][PW / 4];
 #pragma unroll
         for (int tj = 0; tj < TBC; tj++) {
             const int bj = wc + WC * tj;
 #pragma unroll
-            for (int s4 = 0; s4 < 4; s4++) {
-                const double x = rb[4 * s4 + lg][16 * (bj < NB ? bj : 0) + lc];
-                b[tj][s4] = bj != pb ? x : (4 * s4 + lg == lc ? 1.0 : 0.0);
-            }
+            for (int s4 = 0; s4 < PW / 4; s4++) b[tj][s4] = rb[4 * s4 + lg][16 * (bj < NB ? bj : 0) + lc];
         }
 #pragma unroll
         for (int ti = 0; ti < TBR; ti++) {
             const int bi = wr + 2 * ti;
-            double a[4];
+            double a[PW / 4];
 #pragma unroll
-            for (int s4 = 0; s4 < 4; s4++) a[s4] = sh.dfac[4 * s4 + lg][16 * (bi < NB ? bi : 0) + lc];
+            for (int s4 = 0; s4 < PW / 4; s4++) a[s4] = sh.dfac[4 * s4 + lg][16 * (bi < NB ? bi : 0) + lc];
 #pragma unroll
-            for (int s4 = 0; s4 < 4; s4++)
+            for (int s4 = 0; s4 < PW / 4; s4++)
 #pragma unroll
                 for (int tj = 0; tj < TBC; tj++)
                     acc[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s4], b[tj][s4], acc[ti][tj], 0, 0, 0);
