@@ -1,6 +1,6 @@
 // Rate constants, chemistry + diffusion right-hand side, Jacobian and Ros2
-// left-hand-side assembly.  One workgroup per layer for the per-layer
-// kernels: the layer's y row and its reaction rates live in LDS, species
+// left-hand-side assembly.  One workgroup per layer or few layers for the
+// per-layer kernels: a layer's y row and its reaction rates live in LDS, species
 // rows are gathered from per-species CSR lists (no atomics, fixed order).
 #include <algorithm>
 
