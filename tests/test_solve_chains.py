@@ -1,7 +1,7 @@
 """The chain solves around every edge of their layout: the 16-species tiles,
 one, two or three columns per lane, waves whose last rows or all rows lie past
 the block, chains shorter than, as long as and longer than the loads in flight
-(1, 2, 3, 4 and 8 layers), without and with a refinement (which adds into the
+(1, 2 and 4 layers), without and with a refinement (which adds into the
 solution), against a dense solve in float64.
 
 Tolerance: as for the factorisation, condition numbers of at most a few

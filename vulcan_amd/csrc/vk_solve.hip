@@ -64,8 +64,8 @@ __global__ void k_zero_int(int n, int *__restrict__ p) {
 // load), has no exit but its end and no access that a branch skips (the count
 // of what is in flight stays known); rows past the block and steps past the
 // end are buffer accesses out of range, which load zero and store nothing.
-// 256 columns of 80 to 200 layers, 93 species: 675 -> 512 us a sweep (3.7 ->
-// 4.8 TB/s; the kernel before moved its buffers down and so had one layer in
+// 256 columns of 80 to 200 layers, 93 species: 675 -> 482 us a sweep (3.7 ->
+// 5.1 TB/s; the kernel before moved its buffers down and so had one layer in
 // flight); 80 columns of 100 to 150 layers, 150 species: 565 -> 465 us (160
 // chains leave 96 CUs idle); one column of 60 layers, 30 species: 22 -> 18 us
 // (0.45 us a step: barrier, LDS round trip and 70 instructions of one wave).
@@ -84,17 +84,18 @@ __device__ __forceinline__ double add_pair(double v) {
 }
 
 // W CH >= 16 NB rows, 64 C >= 16 NB columns; C <= 16 (NB - 1) + 1, so a
-// lane's columns always fit in the block.  16 waves at no more than 128
-// registers keep DEP layers of one chain in flight on a CU; blocks of up to 64
-// species have too few rows for that many.  DEP steps' loads and stores stay
+// lane's columns always fit in the block.  Eight waves at no more than 128
+// registers put two chains on a CU (one of 16 waves with 3 layers in flight:
+// 512 against 482 us below); from 97 species a layer's share takes 16 waves,
+// and a CU holds one chain.  DEP steps' loads and stores stay
 // below the 63 a wave can track.
 template <int NB>
 struct Sweep {
     static constexpr int C = NB <= 4 ? 1 : (NB <= 8 ? 2 : 3);
-    static constexpr int W = NB == 1 ? 4 : (NB <= 4 ? 8 : 16);
+    static constexpr int W = NB == 1 ? 4 : (NB <= 6 ? 8 : 16);
     static constexpr int CH = 16 * NB / W;
     static constexpr int G = CH <= 4 ? W : (CH <= 8 ? 8 : 4);    // lanes per species: CH G <= 64
-    static constexpr int DEP = NB <= 4 ? 4 : (NB <= 6 ? 3 : (NB <= 8 ? 2 : 1));
+    static constexpr int DEP = NB <= 4 ? 4 : (NB <= 8 ? 2 : 1);
     static constexpr int NTH = 64 * W, MINW = NB <= 4 ? 2 : 4;
     static constexpr int RP = 64 * C + 8;                        // row pitch: G rows on different banks
     static_assert(W * CH == 16 * NB && 64 * C >= 16 * NB && C <= 16 * (NB - 1) + 1 && CH * G <= 64 && W % G == 0,
