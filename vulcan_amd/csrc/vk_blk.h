@@ -2,6 +2,8 @@
 // Gauss-Jordan inversion on FP64 MFMA tiles (chain factorisation and cyclic
 // reduction) and the slab products of the cyclic-reduction updates.
 #pragma once
+#include <cstddef>
+
 #include "vk_internal.h"
 
 namespace {
@@ -56,13 +58,11 @@ template <int NB>
 constexpr int DIAG_PW = NB <= 3 || blk_nt(NB) > NT ? 8 : 16;
 
 template <int NB>
-struct BlkShared {
+struct alignas(16) BlkShared {
     static constexpr int N16 = 16 * NB;
     // above 128 rows the panel wave parks its accumulator tiles here during
     // the panel (its registers then hold the panel alone)
     static constexpr bool PARK = NB >= 9;
-    int info;
-    int refused;                      // a diagonal pivot was refused (blk_invert_diag)
     union {
         struct {                      // blk_invert
             double pan[2][16][N16 + 1];   // panel columns, [k][row], double-buffered by panel parity
@@ -80,7 +80,17 @@ struct BlkShared {
             double diag[N16];             // the block's diagonal as given
         };
     };
+    // behind the arrays, whose 16-byte accesses need the alignment: in front of
+    // them they cost the searched inversion of up to 32 rows the fourth
+    // workgroup of a CU (140 registers for 106: every chain of 512 columns of
+    // 30 species searched, 1.75 ms against 1.02) and that of 64 rows a tenth
+    // of its time
+    int info;
+    int refused;                      // a diagonal pivot was refused (blk_invert_diag)
 };
+static_assert(offsetof(BlkShared<6>, pan) % 16 == 0 && offsetof(BlkShared<6>, prow) % 16 == 0 &&
+                  offsetof(BlkShared<10>, park) % 16 == 0,
+              "arrays of the searched inversion on 16 bytes");
 
 template <int CTRL>
 __device__ __forceinline__ unsigned long long dpp_u64(unsigned long long v) {
