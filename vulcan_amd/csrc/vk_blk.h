@@ -10,7 +10,7 @@ namespace {
 
 constexpr int NT = 256;
 
-// Threads of a blocked-inversion workgroup: 4 waves up to 112 rows, 8 waves
+// Threads of a blocked-inversion workgroup: 4 waves up to 96 rows, 8 waves
 // above (the accumulator tiles of 128-160 rows would not fit 4 waves'
 // registers), with the waves in a 2 x (waves / 2) grid over the tiles.
 constexpr int blk_nt(int nb) { return nb >= 7 ? 512 : 256; }
@@ -632,6 +632,8 @@ enum BlkSearch {
 // entry of the block's output.
 constexpr unsigned long long BLK_MARK = 0x7ff4756c63616e00ull;
 
+__device__ __forceinline__ void blk_mark(double *X) { *(volatile unsigned long long *)X = BLK_MARK; }
+
 __device__ __forceinline__ bool blk_marked(const double *X) {
     return *(const volatile unsigned long long *)X == BLK_MARK;
 }
@@ -648,7 +650,7 @@ __device__ __forceinline__ bool blk_invert_schur(int ni, const double *__restric
         blk_load_schur<NB>(acc, ni, Dl, cl, Xn, cn, cl2, Xn2, cn2);
         if (blk_invert_diag<NB>(acc, ni, X, sh)) return true;
         if constexpr (SEARCH == BLK_SEARCH_MARK) {
-            if (threadIdx.x == 0) *(volatile unsigned long long *)X = BLK_MARK;
+            if (threadIdx.x == 0) blk_mark(X);
             return false;
         }
     }

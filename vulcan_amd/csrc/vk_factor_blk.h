@@ -1,23 +1,27 @@
 // Block-Thomas factorisation, blocked Gauss-Jordan variants (factor
 // variants 1 and 2: one or two resident workgroups per CU).  The inversion
-// itself is blk_invert (panels of 16 pivots on one wave, rank-16 Schur
-// updates on FP64 MFMA).  Included by vk_factor_blk1.hip and
-// vk_factor_blk2.hip, one translation unit per occupancy.
+// itself is blk_invert_diag (the diagonal as pivots, panels of 8 or 16 on every
+// wave) or, for blocks that refuse it, blk_invert (panels of 16 searched pivots
+// on one wave), both with Schur updates on FP64 MFMA.  Included by
+// vk_factor_blk1.hip and vk_factor_blk2.hip, one translation unit per occupancy.
 #pragma once
 #include "vk_blk.h"
 
 namespace {
 
-// 8-wave workgroups (blocks above 112 rows) run one per CU
+// 8-wave workgroups (blocks above 96 rows) run one per CU
 // (order: the chain each workgroup runs, 2c + side; null = blockIdx.x)
 //
-// SEARCH: a chain runs with diagonal pivots (BLK_SEARCH_MARK) up to the first
-// block that refuses them, which it marks; a second launch
-// (BLK_SEARCH_ONLY) runs the rest of such chains with searched pivots.  Both
-// inversions in one kernel do not fit the registers above 128 rows (100 to
-// 290 spilled registers in the chain's loop; 13.3 -> 18.3 ms for nine
-// 150-species columns), and the second launch costs the chains that have
-// nothing left a few microseconds.
+// A chain takes the diagonal as pivots up to the first block that refuses it
+// and searches them from there on: a batch with refusing chains lasts as long
+// as its slowest chain.  In two launches (BLK_SEARCH_MARK, BLK_SEARCH_ONLY) the
+// searching chains start when all the others have ended: one refusing chain
+// of 256 columns, 93 species, 5.77 ms against 3.51 (every chain searched 3.81),
+// of one column of 150 species 12.7 against 8.0.  Only where the diagonal
+// alone leaves registers for two workgroups a CU and more chains than CUs
+// want them (97 to 112 species; launch_blk) two launches are the better
+// choice: 256 columns of 112 species 4.27 against 5.53 ms, with one refusing
+// chain 8.6 against 7.0 (every chain searched 8.3).
 template <int NB, int SEARCH, int MINW>
 __global__ void __launch_bounds__(blk_nt(NB), blk_nt(NB) > NT ? 1 : MINW) k_factor_blk(int ni, const int *__restrict__ off,
                                                     const int *__restrict__ order, const double *__restrict__ D,
@@ -46,9 +50,7 @@ __global__ void __launch_bounds__(blk_nt(NB), blk_nt(NB) > NT ? 1 : MINW) k_fact
             if (blk_marked(Dinv + (size_t)(l0 + j0 + dir * u) * nn)) atomicMin(&sh.refused, u);
         __syncthreads();
         t = sh.refused;
-        if (t >= cnt) return;
-    }
-    if constexpr (SEARCH == BLK_SEARCH_MARK) {
+    } else {
         // the inverse stays in the accumulators for the next block's Schur term
         f64x4 acc[BlkGrid<NB>::TBR][BlkGrid<NB>::TBC];
         for (; t < cnt; ++t) {
@@ -58,22 +60,25 @@ __global__ void __launch_bounds__(blk_nt(NB), blk_nt(NB) > NT ? 1 : MINW) k_fact
             else
                 blk_next_schur<NB>(acc, ni, D + l * nn, cown + l * ni, cprev + (size_t)((long)l - dir) * ni);
             if (!blk_invert_diag<NB>(acc, ni, Dinv + l * nn, sh)) {
-                if (threadIdx.x == 0) *(volatile unsigned long long *)(Dinv + l * nn) = BLK_MARK;
+                if constexpr (SEARCH == BLK_SEARCH_HERE) break;
+                if (threadIdx.x == 0) blk_mark(Dinv + l * nn);
                 return;
             }
         }
-        return;
     }
-    if (threadIdx.x == 0) sh.info = 0;
-    for (; t < cnt; ++t) {
-        const int j = j0 + dir * t;
-        const size_t l = (size_t)l0 + j, lp = (size_t)((long)l - dir);
-        if (!blk_invert_schur<NB, SEARCH>(ni, D + l * nn, cown + l * ni, t > 0 ? Dinv + lp * nn : nullptr,
-                                          t > 0 ? cprev + lp * ni : nullptr, nullptr, nullptr, nullptr, Dinv + l * nn,
-                                          sh, j + 1))
-            return;
+    if (t >= cnt) return;
+    if constexpr (SEARCH != BLK_SEARCH_MARK) {
+        if (threadIdx.x == 0) sh.info = 0;
+        for (; t < cnt; ++t) {
+            const int j = j0 + dir * t;
+            const size_t l = (size_t)l0 + j, lp = (size_t)((long)l - dir);
+            f64x4 acc[BlkGrid<NB>::TBR][BlkGrid<NB>::TBC];
+            blk_load_schur<NB>(acc, ni, D + l * nn, cown + l * ni, t > 0 ? Dinv + lp * nn : nullptr,
+                               t > 0 ? cprev + lp * ni : nullptr, nullptr, nullptr, nullptr);
+            blk_invert<NB>(acc, ni, Dinv + l * nn, sh, j + 1);
+        }
+        if (threadIdx.x == 0 && info && sh.info) atomicCAS(&info[c], 0, sh.info);
     }
-    if (SEARCH != BLK_SEARCH_MARK && threadIdx.x == 0 && info && sh.info) atomicCAS(&info[c], 0, sh.info);
 }
 
 template <int NB, int SEARCH, int MINW>
@@ -99,10 +104,15 @@ __global__ void __launch_bounds__(blk_nt(NB), blk_nt(NB) > NT ? 1 : MINW) k_fact
 template <int N, int MINW>
 void launch_blk(int ni, int ncols, const int *off, const int *order, const double *D, const double *Lsub,
                 const double *Usup, double *Dinv, int *info, const vk_colstate *st, hipStream_t s) {
-    hipLaunchKernelGGL((k_factor_blk<N, BLK_SEARCH_MARK, MINW>), dim3(2 * ncols), dim3(blk_nt(N)), 0, s, ni, off, order,
-                       D, Lsub, Usup, Dinv, info, st);
-    hipLaunchKernelGGL((k_factor_blk<N, BLK_SEARCH_ONLY, MINW>), dim3(2 * ncols), dim3(blk_nt(N)), 0, s, ni, off, order,
-                       D, Lsub, Usup, Dinv, info, st);
+    auto chains = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(2 * ncols), dim3(blk_nt(N)), 0, s, ni, off, order, D, Lsub, Usup, Dinv, info, st);
+    };
+    if (N == 7 && 2 * ncols > vk_device_cus()) {
+        chains(k_factor_blk<7, BLK_SEARCH_MARK, MINW>);
+        chains(k_factor_blk<7, BLK_SEARCH_ONLY, MINW>);
+    } else {
+        chains(k_factor_blk<N, BLK_SEARCH_HERE, MINW>);
+    }
     hipLaunchKernelGGL((k_factor_blk_mid<N, BLK_SEARCH_MARK, MINW>), dim3(ncols), dim3(blk_nt(N)), 0, s, ni, off, D,
                        Lsub, Usup, Dinv, info, st);
     hipLaunchKernelGGL((k_factor_blk_mid<N, BLK_SEARCH_ONLY, MINW>), dim3(ncols), dim3(blk_nt(N)), 0, s, ni, off, D,
