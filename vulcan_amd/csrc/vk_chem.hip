@@ -430,7 +430,7 @@ __global__ void __launch_bounds__(BLK) k_rhs(
 // them once for both (a slot's values of the layers side by side in LDS).
 // 93 species, 620 pairs: 36 000 layers 1695 -> 1310 us (1435 with one layer a
 // workgroup; the vector cache waits on L2 for four fifths of it, the 2.7 GB of
-// sectors it touches take 0.4 ms), 1700 layers 131 -> 87 us, 150 layers
+// sectors it touches take 0.4 ms), 2048 layers 139 -> 76 us, 150 layers
 // 39 -> 22 us.
 // ---------------------------------------------------------------------------
 
@@ -461,8 +461,9 @@ __device__ __forceinline__ void add_term(double (&J)[LG], bool first, int t, con
     for (int a = 0; a < LG; a++) J[a] = first ? c * d[a] : J[a] + c * d[a];
 }
 
-template <int LG>
-__global__ void __launch_bounds__(BLK *LG, 4) k_jac_lhs(
+// NTH threads for the LG layers, WAVES a SIMD
+template <int LG, int NTH, int WAVES>
+__global__ void __launch_bounds__(NTH, WAVES) k_jac_lhs(
     int L, int ni, int npairs, int nslot, int nlight, int nheavy, int njac, const int *__restrict__ off,
     const int *__restrict__ layer_col, const int *__restrict__ reac, const int *__restrict__ prod,
     const int4 *__restrict__ slot_tab, const int4 *__restrict__ jac_ent, const int4 *__restrict__ jac_light,
@@ -485,12 +486,12 @@ __global__ void __launch_bounds__(BLK *LG, 4) k_jac_lhs(
         any = any || on[a];
     }
     if (!any) return;
-    for (int q = threadIdx.x; q < ni + 2; q += BLK * LG)
+    for (int q = threadIdx.x; q < ni + 2; q += NTH)
 #pragma unroll
         for (int a = 0; a < LG; a++)
             yl[LG * q + a] = q < ni ? y[(size_t)x[a].l * ni + q] : (q == ni ? M[x[a].l] : 1.0);
     __syncthreads();   // the slot derivatives read yl
-    for (int s = threadIdx.x; s < nslot; s += BLK * LG) {
+    for (int s = threadIdx.x; s < nslot; s += NTH) {
         const int4 e = slot_tab[s];
         const int p = VK_IX(e.x, npairs, VK_SITE_SLOTPAIR);
         double kf[LG], kb[LG], d[LG];
@@ -540,7 +541,7 @@ __global__ void __launch_bounds__(BLK *LG, 4) k_jac_lhs(
         else if (xa.j == xa.nz - 1 && ca.vm && mol && atm.top_flux && esc_any(atm)) xmode = 1;
         diag[a].xmode = xmode;
         // each layer's species on threads of their own
-        for (int i = (int)threadIdx.x - BLK * a; i < ni; i += BLK * LG) {
+        for (int i = (int)threadIdx.x - NTH / LG * a; i < ni; i += NTH) {
             if (i < 0) continue;
             LhsDiff r = lhs_diff(ca, xa.j, i, ysm, ys0, ysp, ms[i], alpha[i], mol != 0);
             dg0[i] = r.d0;
@@ -568,8 +569,12 @@ __global__ void __launch_bounds__(BLK *LG, 4) k_jac_lhs(
     // write_zeros: the integrator clears its blocks once and skips them): the
     // few long term lists (jac_ent[0, nheavy): the list is sorted by term
     // count) by threads of their own, the others in one nearly coalesced pass
-    // in the order of the dense index.  With few layers the entries of a
-    // layer are split over the grid's y dimension (each workgroup forms the
+    // in the order of the dense index.  With the zeros that pass runs over the
+    // dense index itself and writes whole lines where there are many layers
+    // (the zeros in a pass behind the entries: 32 768 layers of 150 species 4.11
+    // ms for 3.15); the lanes on zeros then wait for the others, so few layers
+    // keep the pass behind (64 layers 38 us for 46).  With few layers the entries
+    // of a layer are split over the grid's y dimension (each workgroup forms the
     // layer's shared terms itself).
     auto store = [&](int e, const double (&J)[LG], bool dg) {
         e = VK_IX(e, nn, VK_SITE_DENSE);
@@ -583,7 +588,7 @@ __global__ void __launch_bounds__(BLK *LG, 4) k_jac_lhs(
             if (on[a]) D[(size_t)x[a].l * nn + e] = val;
         }
     };
-    const int e0 = threadIdx.x + blockIdx.y * BLK * LG, es = BLK * LG * gridDim.y;
+    const int e0 = threadIdx.x + blockIdx.y * NTH, es = NTH * gridDim.y;
     for (int q = e0; q < nheavy; q += es) {
         const int4 en = jac_ent[q];       // (dense index, first term, end of terms, row)
         double J[LG];
@@ -600,8 +605,7 @@ __global__ void __launch_bounds__(BLK *LG, 4) k_jac_lhs(
         for (; u < en.z; u++) add_term<LG>(J, false, jac_tp[VK_IX(u, njac, VK_SITE_TERM)], dv, nslot);
         store(en.x, J, en.x == en.w * (ni + 1));
     }
-#pragma unroll 2
-    for (int q = e0; q < nlight; q += es) {
+    auto light = [&](int q) {
         const int4 en = jac_light[q];
         const int nt = en.x >> 16 & 15;
         int t[VK_JAC_LIGHT];
@@ -614,13 +618,26 @@ __global__ void __launch_bounds__(BLK *LG, 4) k_jac_lhs(
         for (int m = 2; m < VK_JAC_LIGHT; m++)
             if (m < nt) add_term<LG>(J, false, t[m], dv, nslot);
         store(en.x & 0xffff, J, en.x >> 20);
-    }
-    if (write_zeros)
-        for (int e = e0; e < nn; e += es)
-            if (jac_emap[e] < 0)
+    };
+    auto zero = [&](int e) {
+        if (jac_emap[e] == VK_JAC_ZERO)
 #pragma unroll
-                for (int a = 0; a < LG; a++)
-                    if (on[a]) D[(size_t)x[a].l * nn + e] = 0.0;
+            for (int a = 0; a < LG; a++)
+                if (on[a]) D[(size_t)x[a].l * nn + e] = 0.0;
+    };
+    if (LG > 1 && write_zeros) {
+#pragma unroll 2
+        for (int e = e0; e < nn; e += es) {
+            const int q = jac_emap[e];
+            if (q >= 0) light(q);
+            else zero(e);
+        }
+        return;
+    }
+#pragma unroll 2
+    for (int q = e0; q < nlight; q += es) light(q);
+    if (write_zeros)
+        for (int e = e0; e < nn; e += es) zero(e);
 }
 
 }  // namespace
@@ -700,20 +717,32 @@ int vk_launch_jac_lhs(const vk_plan *plan, const vk_columns *cols, const vk_atm 
         }
     }
     const int ncu = vk_device_cus();
-    auto launch = [&](auto kernel, int layers, int gy) {
-        hipLaunchKernelGGL(kernel, dim3((cols->L + layers - 1) / layers, gy), dim3(BLK * layers), jac_smem(plan, layers),
-                           s, cols->L, plan->ni, plan->npairs, plan->nslot, plan->njlight, plan->njheavy, plan->njac,
+    auto launch = [&](auto kernel, int layers, int threads, int gy) {
+        hipLaunchKernelGGL(kernel, dim3((cols->L + layers - 1) / layers, gy), dim3(threads), jac_smem(plan, layers), s,
+                           cols->L, plan->ni, plan->npairs, plan->nslot, plan->njlight, plan->njheavy, plan->njac,
                            cols->d_off, cols->d_layer_col, plan->reac, plan->prod, plan->slot_tab, plan->jac_ent,
                            plan->jac_light, plan->jac_emap, plan->jac_tp, plan->ms, plan->alpha, a, y, k, M, mode, mol,
                            dtc, ysum, st, D, Lsub, Usup, (int)write_zeros);
     };
-    // two layers a workgroup where two such workgroups fit a CU's 160 KB and
-    // every CU still gets several; fewer layers than twice the CUs: each
-    // layer's entries over up to 4 workgroups
-    if (jac_smem(plan, 2) <= 80 * 1024 && cols->L >= 12 * ncu)
-        launch(k_jac_lhs<2>, 2, 1);
+    // Up to one layer a CU: one layer a workgroup, its entries over up to 4 of
+    // them.  Beyond, two layers a workgroup (448 layers of 150 species 53
+    // against 65 us, 93 species 40 against 43) where two such workgroups fit a
+    // CU's 160 KB.  What a small network's layer takes is latency, so with six
+    // layers a CU and more its two layers run on 256 threads where the LDS then
+    // holds as many waves as with 512 (four workgroups) or more (six), for the
+    // layers in flight: 32 768 layers, 512 threads against 256 of four and of six
+    // workgroups: 30 species 445, 308, 267 us, 40 species 566, 417, 351, 61
+    // species 808, 714, 751, 93 species (three workgroups) 1217, 1325, 1368; 61
+    // species, 1024 layers 37 against 44 and 2048 layers 57 against 51.
+    const size_t two = jac_smem(plan, 2);
+    if (two > 80 * 1024 || cols->L <= ncu)
+        launch(k_jac_lhs<1, BLK, 4>, 1, BLK, ncu > 0 ? std::max(1, std::min(4, 2 * ncu / std::max(cols->L, 1))) : 1);
+    else if (two > 160 * 1024 / 4 || cols->L < 6 * ncu)
+        launch(k_jac_lhs<2, 2 * BLK, 4>, 2, 2 * BLK, 1);
+    else if (two > 160 * 1024 / 6)
+        launch(k_jac_lhs<2, BLK, 4>, 2, BLK, 1);
     else
-        launch(k_jac_lhs<1>, 1, ncu > 0 ? std::max(1, std::min(4, 2 * ncu / std::max(cols->L, 1))) : 1);
+        launch(k_jac_lhs<2, BLK, 6>, 2, BLK, 1);
     VK_CHECK(hipGetLastError());
     return 0;
 }

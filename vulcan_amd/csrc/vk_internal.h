@@ -38,6 +38,9 @@ __host__ __device__ inline int vk_jac_pack(int slot, int coef) { return (slot <<
 __host__ __device__ inline int vk_jac_slot(int w) { return w >> 8; }
 __host__ __device__ inline double vk_jac_coef(int w) { return (double)((int)((unsigned)w << 24) >> 24); }
 
+// in place of an entry of jac_light: more than VK_JAC_LIGHT terms, a structural zero
+constexpr int VK_JAC_HEAVY = -1, VK_JAC_ZERO = -2;
+
 // an entry of jac_light: dense index, term count, on the diagonal
 static_assert(VK_NI_MAX * VK_NI_MAX <= 1 << 16 && VK_JAC_LIGHT < 16, "fields of vk_light_pack");
 __host__ __device__ inline int vk_light_pack(int e, int nt, bool diag) { return e | nt << 16 | (int)diag << 20; }
@@ -72,7 +75,7 @@ struct vk_plan {
     int *jac_map, *jac_ptr, *jac_slot;
     int njent;                 // entries with chemical terms plus the diagonal
     int4 *jac_ent;             // (dense index, first term, end of terms, row), longest term lists first
-    int *jac_emap;             // dense index -> -1 where the block has a structural zero, else 0
+    int *jac_emap;             // dense index -> entry of jac_light, VK_JAC_HEAVY or VK_JAC_ZERO
     int njlight;               // entries with at most VK_JAC_LIGHT terms, by dense index:
     int4 *jac_light;           // (vk_light_pack, first term, its first two packed terms)
     int4 *slot_tab;            // (pair, vk_side_pack of its reactants and its products, species) of a derivative slot

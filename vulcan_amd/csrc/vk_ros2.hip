@@ -532,14 +532,15 @@ extern "C" int vk_plan_create(const vk_network_desc *n, vk_plan **out) {
                          [](const int4 &x, const int4 &y) { return (x.z - x.y) > (y.z - y.y); });
         p->njent = (int)ent.size();
         p->njheavy = 0;
-        std::vector<int> emap((size_t)n->ni * n->ni, -1);
-        for (int q = 0; q < p->njent; q++) {
+        for (int q = 0; q < p->njent; q++)
             if (ent[q].z - ent[q].y > VK_JAC_LIGHT) p->njheavy = q + 1;
-            emap[ent[q].x] = 0;
-        }
+        light.assign(ent.begin() + p->njheavy, ent.end());
+        std::sort(light.begin(), light.end(), [](const int4 &x, const int4 &y) { return x.x < y.x; });
+        std::vector<int> emap((size_t)n->ni * n->ni, VK_JAC_ZERO);
+        for (int q = 0; q < p->njheavy; q++) emap[ent[q].x] = VK_JAC_HEAVY;
+        for (size_t q = 0; q < light.size(); q++) emap[light[q].x] = (int)q;
         r = upload(v, &p->jac_ent, ent.data(), ent.size());
         r = r ? r : upload(v, &p->jac_emap, emap.data(), emap.size());
-        light.assign(ent.begin() + p->njheavy, ent.end());
     }
     if (!r) {
         int most = 1;
@@ -572,7 +573,6 @@ extern "C" int vk_plan_create(const vk_network_desc *n, vk_plan **out) {
             else terms[q] = vk_jac_pack(sl, (int)c);
         }
         r = r ? r : upload(v, &p->jac_tp, terms.data(), terms.size());
-        std::sort(light.begin(), light.end(), [](const int4 &x, const int4 &y) { return x.x < y.x; });
         for (int4 &e : light) {
             const int u0 = e.y, nt = e.z - e.y;
             e = make_int4(vk_light_pack(e.x, nt, e.x % n->ni == e.w), u0, nt > 0 ? terms[u0] : 0,
