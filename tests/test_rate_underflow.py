@@ -18,7 +18,7 @@ TOL = 1e-12
 
 
 @gpu
-@pytest.mark.parametrize('layers', [7, 40000])
+@pytest.mark.parametrize('layers', [7, 1409, 2817, 5633, 40000])      # one, two, four and eight layers a workgroup
 def test_rates_of_tiny_factors(layers):
     import torch
     if not torch.cuda.is_available():

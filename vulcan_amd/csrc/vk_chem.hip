@@ -659,11 +659,14 @@ extern "C" int vk_rates(const vk_plan *plan, const vk_columns *cols, const vk_at
     if (!plan || !cols || !atm || !d_k) return VK_EINVAL;
     const int L = cols->L, cu = vk_device_cus();
     // layers per workgroup: the most (their pairs' parameters are read once)
-    // that still leave eight workgroups per CU; below that one layer each, and
-    // its pairs over several workgroups
+    // that leave about three workgroups per CU (93 species, 620 pairs, one, two,
+    // four, eight layers: 1 536 layers 26, 21, 28, 38 us, 3 008 layers 42, 36, 32,
+    // 46, 6 144 layers 76, 60, 54, 51); below that one layer each, and its pairs
+    // over several workgroups, each of which forms what the layer's pairs share,
+    // only to give every CU two (1 024 layers over three 27 us, over one 18)
     int LG = RATE_LAYERS;
-    while (LG > 1 && L < 8 * cu * LG) LG /= 2;
-    const int split = LG > 1 ? 1 : (plan->npairs + BLK - 1) / BLK;
+    while (LG > 1 && 4L * L < 11L * cu * LG) LG /= 2;
+    const int split = LG > 1 ? 1 : std::max(1, std::min((plan->npairs + BLK - 1) / BLK, 2 * cu / std::max(L, 1)));
     hipLaunchKernelGGL(k_rates, dim3((L + LG - 1) / LG, split), dim3(BLK), 0, S(stream), L, LG, plan->npairs, plan->ni,
                        plan->kind, plan->par, plan->rev, plan->reac, plan->prod, plan->nasa9, atm->Tco, atm->M,
                        atm->tau, d_k);
