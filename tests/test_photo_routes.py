@@ -1,0 +1,59 @@
+"""Radiative transfer of batches whose size alone moves them to other kernels,
+against their first two columns alone, bit for bit: the photolysis rates of many
+layers with few and with many bins."""
+import numpy as np
+import pytest
+
+gpu = pytest.mark.gpu
+
+
+def _update(torch, nz, nb, period):
+    """Two updates of columns whose layers repeat every `period`; the rows of the
+    first and of the last two columns."""
+    from vulcan_amd import photo as P
+    from vulcan_amd import workloads as W
+    from vulcan_amd.device import DeviceColumns, DevicePlan
+    net = W.small_network()
+    rng = np.random.default_rng(nb)
+    nabs, nbr = 5, 18
+    tab = P.PhotoTables(bins=np.linspace(100., 300., nb), din12=max(1, nb // 3), sflux_top=10.0 ** rng.uniform(2, 5, nb),
+                        abs_sp=[2, 7, 11, 20, 3], abs_T=[-1] * nabs, cross=10.0 ** rng.uniform(-21, -18, (nabs, nb)),
+                        cross_T=np.zeros((0, 0, nb)), scat_sp=[1, 5], cross_scat=10.0 ** rng.uniform(-25, -22, (2, nb)),
+                        br_col=[2 * q for q in range(nbr)], br_T=[-1] * nbr, cross_J=10.0 ** rng.uniform(-21, -18, (nbr, nb)),
+                        cross_J_T=np.zeros((0, 0, nb)), dbin1=0.1, dbin2=2., cos_sl=0.669, edd=0.5, f_diurnal=1.,
+                        flux_atol=1.)
+    y = torch.as_tensor(10.0 ** rng.uniform(5, 13, (period, net.ni)), device='cuda')
+    dz = torch.as_tensor(rng.uniform(1e5, 1e6, period), device='cuda')
+    plan, cols = DevicePlan(net), DeviceColumns(nz)
+    ph = P.DevicePhoto(plan, cols, tab)
+    again = -(-cols.L // period)
+    yd, dzd = y.repeat(again, 1)[:cols.L].contiguous(), dz.repeat(again)[:cols.L].contiguous()
+    k = torch.zeros((cols.L, net.nr), dtype=torch.float64, device='cuda')
+    for _ in range(2):
+        ph.update(yd, yd / yd.sum(dim=1, keepdim=True), dzd, k, force=True)
+    torch.cuda.synchronize()
+    lay, lev = [(n, sum(nz[:2]) + n, sum(nz[-2:]) + n) for n in (0, 2)]
+    out = []
+    for what, rows in [(w, lev) for w in range(4)] + [(4, lay)]:
+        a = ph.read(what)
+        out += [a[:rows[1]], a[-rows[2]:]]
+    out += [k[:lay[1], :2 * nbr].cpu().numpy(), k[-lay[2]:, :2 * nbr].cpu().numpy()]
+    ph.close()
+    assert (out[-1][:, ::2] > 0).all()
+    return out
+
+
+def _compare(nz, count, nb):
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip('no HIP device')
+    few, many = (_update(torch, nz * n, nb, sum(nz)) for n in (1, count))
+    for a, b in zip(few, many):
+        assert np.array_equal(a, b)
+
+
+@gpu
+@pytest.mark.parametrize('nz,count,nb', [([64, 41], 20, 511), ([64, 41], 20, 512), ([64, 41], 20, 3),
+                                         ([64, 41], 20, 2600), ([64, 41], 11, 2601)])
+def test_rates_of_many_layers(nz, count, nb):
+    _compare(nz, count, nb)

@@ -439,22 +439,27 @@ void launch_photo_rt(const PhotoDev &d, const vk_columns *cols, hipStream_t s) {
 // in 0.65 ms; at four 0.38 ms), so batches take as many layers as LDS holds; a column or two
 // take one, with the branches split over the grid's y dimension to fill the
 // device.
-constexpr int J_NT = 1024, J_LDS = 10400;   // doubles: four layers of 2 600 bins, or one of 8 192
+constexpr int J_NT = 1024, J_LDS = 10400;   // doubles: four layers of 2 600 bins, or one of 10 400
+// Below this many bins a workgroup has 4 waves, for the branches to share them
+// evenly (36 over 16 waves take three rounds of which the last is a quarter
+// full): 30 000 layers of 20, 100, 300 bins 362, 359, 410 -> 297, 299, 342 us, of
+// 700 bins 530 us with 16.
+constexpr int J_SMALL = 512, J_SMALL_NT = 256;
 
 // STAGE: the actinic flux through LDS (spectra beyond J_LDS bins read it from
 // memory for every branch)
-template <int LT, bool STAGE = true>
-__global__ void __launch_bounds__(J_NT) k_photo_J(PhotoDev ph, const int *__restrict__ layer_col, int nr,
+template <int LT, int NTH, bool STAGE = true>
+__global__ void __launch_bounds__(NTH) k_photo_J(PhotoDev ph, const int *__restrict__ layer_col, int nr,
                                                   double *__restrict__ k) {
-    __shared__ double lds[STAGE ? J_LDS : 1];
+    extern __shared__ double lds[];
     const int l0 = LT * blockIdx.x, nb = ph.nbin, nl = min(LT, ph.L - l0);
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = J_NT / 64;
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = NTH / 64;
     const bool due = lane < nl && ph.due[layer_col[l0 + min(lane, nl - 1)]];   // lane: layer
     if (!__any(due)) return;
     const double *af = ph.aflux + (size_t)l0 * nb;
     if constexpr (STAGE) {
 #pragma unroll 8
-        for (int e = threadIdx.x; e < LT * nb; e += J_NT) {
+        for (int e = threadIdx.x; e < LT * nb; e += NTH) {
             const double a = af[min(e, nl * nb - 1)];
             lds[e] = e < nl * nb ? a : 0.0;
         }
@@ -614,18 +619,22 @@ int vk_launch_photo(vk_photo *ph, const vk_plan *plan, const vk_columns *cols, c
         hipLaunchKernelGGL(k_photo_flux, grid, dim3(PT), 0, s, d, cols->d_off);
     }
     const int L = cols->L, ncu = std::max(1, vk_device_cus());
-    if (4 * d.nbin <= J_LDS && L >= 8 * ncu)
-        hipLaunchKernelGGL(k_photo_J<4>, dim3((L + 3) / 4), dim3(J_NT), 0, s, d, cols->d_layer_col, plan->nr, k);
+    auto rates = [&](auto kernel, int layers, int threads, int gy, bool stage) {
+        hipLaunchKernelGGL(kernel, dim3((L + layers - 1) / layers, gy), dim3(threads),
+                           stage ? sizeof(double) * layers * (size_t)d.nbin : 0, s, d, cols->d_layer_col, plan->nr, k);
+    };
+    // about two workgroups per CU, at least a branch per wave
+    const int gy = std::max(1, std::min((d.nbranch + J_NT / 64 - 1) / (J_NT / 64), (2 * ncu + L - 1) / L));
+    if (d.nbin < J_SMALL && L >= 8 * ncu)
+        rates(k_photo_J<4, J_SMALL_NT>, 4, J_SMALL_NT, 1, true);
+    else if (4 * d.nbin <= J_LDS && L >= 8 * ncu)
+        rates(k_photo_J<4, J_NT>, 4, J_NT, 1, true);
     else if (2 * d.nbin <= J_LDS && L >= 4 * ncu)
-        hipLaunchKernelGGL(k_photo_J<2>, dim3((L + 1) / 2), dim3(J_NT), 0, s, d, cols->d_layer_col, plan->nr, k);
-    else {
-        // about two workgroups per CU, at least a branch per wave
-        const int gy = std::max(1, std::min((d.nbranch + J_NT / 64 - 1) / (J_NT / 64), (2 * ncu + L - 1) / L));
-        if (d.nbin <= J_LDS)
-            hipLaunchKernelGGL(k_photo_J<1>, dim3(L, gy), dim3(J_NT), 0, s, d, cols->d_layer_col, plan->nr, k);
-        else
-            hipLaunchKernelGGL((k_photo_J<1, false>), dim3(L, gy), dim3(J_NT), 0, s, d, cols->d_layer_col, plan->nr, k);
-    }
+        rates(k_photo_J<2, J_NT>, 2, J_NT, 1, true);
+    else if (d.nbin <= J_LDS)
+        rates(k_photo_J<1, J_NT>, 1, J_NT, gy, true);
+    else
+        rates(k_photo_J<1, J_NT, false>, 1, J_NT, gy, false);
     hipLaunchKernelGGL(k_photo_change, dim3((nc + 127) / 128), dim3(128), 0, s, nc, d.due, d.change, st);
     VK_CHECK(hipGetLastError());
     return 0;
