@@ -1,6 +1,8 @@
 """Radiative transfer of batches whose size alone moves them to other kernels,
 against their first two columns alone, bit for bit: the photolysis rates of many
-layers with few and with many bins."""
+layers with few and with many bins, and the fluxes of batches with so many bins
+in all that a thread takes one each (short columns, columns whose LDS lets two
+workgroups or one share a CU), beside the next smaller batch that does not."""
 import numpy as np
 import pytest
 
@@ -57,3 +59,11 @@ def _compare(nz, count, nb):
                                          ([64, 41], 20, 2600), ([64, 41], 11, 2601)])
 def test_rates_of_many_layers(nz, count, nb):
     _compare(nz, count, nb)
+
+
+@gpu
+@pytest.mark.parametrize('nz,per_bin,nb', [([8, 5], 64000, 131), ([31, 2], 248000, 700), ([63, 40], 504000, 2588),
+                                           ([213, 200], 180000, 700), ([320, 31], 90000, 1000), ([416, 3], 90000, 2588)])
+@pytest.mark.parametrize('beyond', [0, 1])
+def test_fluxes_of_many_bins(nz, per_bin, nb, beyond):
+    _compare(nz, (per_bin - 1) // (2 * nb) + beyond, nb)

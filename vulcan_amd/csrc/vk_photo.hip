@@ -186,7 +186,7 @@ __global__ void __launch_bounds__(PT) k_photo_flux(PhotoDev ph, const int *__res
 // each before, 15 us (k_photo_layers, bound by reading the cross sections
 // from L2) and 37 us (k_photo_rt, a third of it the serial parts) now; 48
 // columns: 1 125 us each before, 170 and 777 us now (three workgroups per CU
-// by LDS).
+// by LDS).  photo_per_bin says where a thread per bin is the better choice.
 // ---------------------------------------------------------------------------
 
 // every layer's own optical depth (left in the tau row of its lower level)
@@ -425,6 +425,29 @@ __global__ void __launch_bounds__(PT) k_photo_rt(PhotoDev ph, const int *__restr
         atomicMax(&ph.change[c], (unsigned long long)__double_as_longlong(mx));
 }
 
+// Whether a thread per bin (k_photo_tau, k_photo_flux) is faster than
+// k_photo_layers and k_photo_rt: its time is a chain over the layers, 7 us each,
+// until the columns' bins fill the device, which k_photo_rt does with a few
+// hundred.  Short columns leave most of its 32 threads a bin without a layer;
+// from 213 layers its LDS lets two workgroups share a CU, from 320 one.  A thread
+// per bin against the two kernels, us (bins x columns in thousands):
+//   8 layers     50 /  42 (34)     75 /  98 (124)    807 / 2046 (2 588)
+//   16 layers   140 / 131 (124)   260 / 381 (350)    834 / 1407 (1 294)
+//   32 layers   314 / 289 (175)   437 / 431 (259)    947 / 1046 (647)
+//   48 layers   379 / 266 (112)   567 / 494 (207)    932 /  988 (414)
+//   64 layers  1078 / 941 (323)  2020 / 1835 (647)  4481 / 4296 (1 553)
+//   150 layers 1455 / 810 (124)                     7492 / 6317 (1 035)
+//   224 layers 2194 / 1772 (124) 3335 / 3615 (259)  6316 / 7204 (518)
+//   300 layers 2910 / 2454 (124) 3783 / 4068 (210)  8444 / 9951 (518)
+//   330 layers 2599 / 2354 (62)  2813 / 3490 (93)
+//   416 layers 3306 / 2886 (62)  3512 / 4285 (93)   7350 / 14151 (311)
+static bool photo_per_bin(int max_nz, long bins) {
+    if (max_nz > RT_LANES * RT_ROUNDS) return true;
+    if (max_nz < 64) return bins >= 8000L * max_nz;
+    const long per_cu = 160 * 1024 / (long)rt_lds(max_nz);
+    return per_cu <= 2 && bins >= 90000 * per_cu;
+}
+
 template <int R>
 void launch_photo_rt(const PhotoDev &d, const vk_columns *cols, hipStream_t s) {
     hipLaunchKernelGGL((k_photo_rt<R>), dim3((d.nbin + RT_BINS - 1) / RT_BINS, cols->ncols), dim3(PT),
@@ -604,7 +627,7 @@ int vk_launch_photo(vk_photo *ph, const vk_plan *plan, const vk_columns *cols, c
     const int nc = cols->ncols;
     hipLaunchKernelGGL(k_photo_due, dim3((nc + 127) / 128), dim3(128), 0, s, nc, st, force, ini_frq, final_frq,
                        yconv_min, d.last, d.switched, d.due, d.change);
-    if (cols->max_nz <= RT_LANES * RT_ROUNDS) {
+    if (!photo_per_bin(cols->max_nz, (long)d.nbin * nc)) {
         hipLaunchKernelGGL(k_photo_layers, dim3((d.nbin + PT - 1) / PT, (cols->L + TAU_LAYERS - 1) / TAU_LAYERS), dim3(PT),
                            0, s, d, plan->ni, cols->d_layer_col, y, ymix, dz);
         switch ((cols->max_nz + RT_LANES - 1) / RT_LANES) {
