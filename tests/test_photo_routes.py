@@ -67,3 +67,9 @@ def test_rates_of_many_layers(nz, count, nb):
 @pytest.mark.parametrize('beyond', [0, 1])
 def test_fluxes_of_many_bins(nz, per_bin, nb, beyond):
     _compare(nz, (per_bin - 1) // (2 * nb) + beyond, nb)
+
+
+@gpu
+def test_half_a_million_layers():
+    """More groups of eight layers than a grid is long in y (65 535)."""
+    _compare([128, 130], 2040, 5)

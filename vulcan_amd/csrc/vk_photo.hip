@@ -199,9 +199,11 @@ __global__ void __launch_bounds__(PT, 4) k_photo_layers(PhotoDev ph, int ni, con
                                                      const double *__restrict__ y, const double *__restrict__ ymix,
                                                      const double *__restrict__ dz) {
     __shared__ double ny[TAU_SPECIES][TAU_LAYERS], mx[TAU_SPECIES][TAU_LAYERS];   // y dz and ymix
-    const int l0 = TAU_LAYERS * blockIdx.y, nl = min(TAU_LAYERS, ph.L - l0), nb = ph.nbin;
-    const int b = min((int)(blockIdx.x * PT + threadIdx.x), nb - 1);
-    const bool mine = blockIdx.x * PT + threadIdx.x < nb;
+    // one dimension: a grid's y is 65 535 long, half a million layers
+    const int nb = ph.nbin, groups = (nb + PT - 1) / PT;
+    const int l0 = TAU_LAYERS * (blockIdx.x / groups), nl = min(TAU_LAYERS, ph.L - l0);
+    const int bt = PT * (blockIdx.x % groups) + threadIdx.x, b = min(bt, nb - 1);
+    const bool mine = bt < nb;
     bool any = false;
     for (int q = 0; q < nl; q++) any = any || ph.due[layer_col[l0 + q]];
     if (!any) return;
@@ -628,7 +630,7 @@ int vk_launch_photo(vk_photo *ph, const vk_plan *plan, const vk_columns *cols, c
     hipLaunchKernelGGL(k_photo_due, dim3((nc + 127) / 128), dim3(128), 0, s, nc, st, force, ini_frq, final_frq,
                        yconv_min, d.last, d.switched, d.due, d.change);
     if (!photo_per_bin(cols->max_nz, (long)d.nbin * nc)) {
-        hipLaunchKernelGGL(k_photo_layers, dim3((d.nbin + PT - 1) / PT, (cols->L + TAU_LAYERS - 1) / TAU_LAYERS), dim3(PT),
+        hipLaunchKernelGGL(k_photo_layers, dim3((d.nbin + PT - 1) / PT * ((cols->L + TAU_LAYERS - 1) / TAU_LAYERS)), dim3(PT),
                            0, s, d, plan->ni, cols->d_layer_col, y, ymix, dz);
         switch ((cols->max_nz + RT_LANES - 1) / RT_LANES) {
         case 1: case 2: case 3: launch_photo_rt<3>(d, cols, s); break;
@@ -668,6 +670,7 @@ extern "C" int vk_photo_update(vk_photo *p, const vk_plan *plan, const vk_column
                                int ini_frq, int final_frq, double yconv_min, void *stream) {
     if (!p || !plan || !cols || !d_y || !d_ymix || !d_dz || !d_k) return VK_EINVAL;
     if (!force && (!d_st || ini_frq < 1 || final_frq < 1)) return VK_EINVAL;
+    // a limit of this entry alone: the kernels, and the integration's own refresh, take longer spectra
     if ((size_t)p->d.nbin * sizeof(double) > 64 * 1024) return VK_ETOOBIG;
     return vk_launch_photo(p, plan, cols, d_y, d_ymix, d_dz, d_k, d_st, force, ini_frq, final_frq, yconv_min,
                            (hipStream_t)stream);
