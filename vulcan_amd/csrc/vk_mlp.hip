@@ -33,15 +33,22 @@ __device__ __forceinline__ void store_tile(const f32x16 &acc, int M, int N, int 
     const int col = n0 + (lane & 31);
     if (col >= N) return;
     const float bc = bias ? bias[col] : 0.0f;
+    float *cp = C + (long)(m0 + 4 * (lane >> 5)) * ldc + col;
+    if (!accumulate && !Yact) {
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            const int r = 8 * (q >> 2) + (q & 3);
+            if (m0 + 4 * (lane >> 5) + r < M) cp[(long)r * ldc] = bias ? acc[q] + bc : acc[q];
+        }
+        return;
+    }
 #pragma unroll
     for (int q = 0; q < 16; q++) {
-        const int row = m0 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
+        const int r = 8 * (q >> 2) + (q & 3), row = m0 + 4 * (lane >> 5) + r;
         if (row < M) {
-            float v = acc[q];
-            if (bias) v += bc;
-            float *cp = C + (long)row * ldc + col;
-            if (accumulate) v += *cp;
-            *cp = v;
+            float v = bias ? acc[q] + bc : acc[q];
+            if (accumulate) v += cp[(long)r * ldc];
+            cp[(long)r * ldc] = v;
             if (Yact) Yact[(long)row * ldy + col] = f2bf(silu(v));
         }
     }
@@ -113,8 +120,9 @@ __global__ void __launch_bounds__(256) k_gemm_any(int M, int N, int K, const uns
 // 1024 x 1024 layers 123 -> 11 us (64 of the 256 CUs worked), the 1024 x
 // 13 950 head 198 -> 38 us, its weight gradient 157 -> 49 us, a training step
 // of the 307 -> 4 x 1024 -> 13 950 network 3.60 -> 0.47 ms.  The head's input
-// gradient (k = 13 950 on 32 x 32 tiles, 1 744 dependent MFMAs, 70 us) is
-// bound by that chain.
+// gradient (k = 13 950 on 32 x 32 tiles, 70 us) is 1 744 dependent MFMAs on one
+// wave of four; at 32 cycles each these are 23 us, and a chunk's barrier, its
+// LDS reads and the staging by the same wave lie between them.
 // ---------------------------------------------------------------------------
 struct GemmArgs {
     int M, N, K;
@@ -411,14 +419,21 @@ extern "C" int vk_mlp_gemm(int M, int N, int K, const void *d_A, long sam, long 
                            long ldy, void *stream) {
     if (M <= 0 || N <= 0 || K <= 0 || !d_A || !d_B || !d_C) return VK_EINVAL;
     hipStream_t s = (hipStream_t)stream;
-    // the tiled kernel where each operand has a unit stride
+    // The tiled kernel where each operand has a unit stride.  Its chunks are 64 or
+    // 128 deep; with a product less deep, many outputs are faster through
+    // k_gemm_any, 32 at a time (1024 x 13 950 outputs, k = 8, 32, 48, 63, 64, 96: 20,
+    // 23, 32, 34, 34, 46 us against 36, 37, 38, 40, 30, 41; 1024 x 1024, k = 32, 48:
+    // 9.8, 10.6 against 9.0, 8.9).
     const bool ak = sak == 1, am = sam == 1, bk = sbk == 1, bn = sbn == 1;
-    if ((ak || am) && (bk || bn)) {
+    const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64), t128 = (long)((M + 127) / 128) * ((N + 63) / 64);
+    const int ncu = vk_device_cus();
+    const bool shallow = K < 64 && t64 >= 2L * ncu && (M + TM - 1) / TM <= 65535;
+    if ((ak || am) && (bk || bn) && !shallow) {
         const GemmArgs g = {M, N, K, (const unsigned short *)d_A, (const unsigned short *)d_B, ak ? sam : sak,
                             bk ? sbn : sbk, d_C, ldc, d_bias, accumulate, (unsigned short *)d_Yact, ldy};
-        const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64), t128 = (long)((M + 127) / 128) * ((N + 63) / 64);
-        const int ncu = vk_device_cus();
-        if (t128 >= 2L * ncu) launch_gemm<128, 64, 64, 32, 64>(g, ak, bk, s);
+        // 128 rows a tile only where at most an eighth of them lies past the
+        // last row (64 x 262 144 outputs, k = 128: FIGM)
+        if (t128 >= 2L * ncu && 8 * (2 * t128 - t64) <= t64) launch_gemm<128, 64, 64, 32, 64>(g, ak, bk, s);
         else if (t64 >= ncu) launch_gemm<64, 64, 32, 32, 64>(g, ak, bk, s);
         else launch_gemm<32, 32, 32, 32, 128>(g, ak, bk, s);
     } else {
