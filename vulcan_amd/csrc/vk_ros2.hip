@@ -555,8 +555,9 @@ extern "C" int vk_plan_create(const vk_network_desc *n, vk_plan **out) {
         auto bytes = [&](const int *t) {
             unsigned w = 0;
             for (int q = 0; q < 4; q++) {
-                const int f = t[q] == -2 ? n->ni + 1 : (t[q] == -1 ? n->ni : t[q]);
-                w |= (unsigned)(f < 0 || f > n->ni + 1 ? 255 : f) << 8 * q;
+                // no species: an index beyond the amounts (vk_debug_checks)
+                const int f = t[q] >= n->ni || t[q] < -2 ? 255 : (t[q] == -2 ? n->ni + 1 : (t[q] == -1 ? n->ni : t[q]));
+                w |= (unsigned)f << 8 * q;
             }
             return w;
         };
