@@ -138,3 +138,66 @@ def test_one_refusing_chain_costs_no_second_pass(variant, ni):
             best[q] = min(best[q], a.elapsed_time(b))
     print('every chain refuses %.3f ms, one %.3f ms' % tuple(best), flush=True)
     assert best[1] < 1.15 * best[0]
+
+
+@gpu
+@pytest.mark.parametrize('every', [0, 2, 7, 9, 40])
+@pytest.mark.parametrize('ni', [17, 97])
+def test_cyclic_reduction_with_some_refusing(ni, every):
+    """Refusals among the blocks that level 0 eliminates, none, fewer than one in
+    eight or more (the later levels then search at once), and among the others
+    too; columns of even and odd length, more blocks a launch than CUs."""
+    from test_factor_pivots import TOL, _dense, _system
+    nz = [40, 41, 2, 3] + [9] * 56
+    torch, lib, plan, cols = _setup(ni, nz)
+    from vulcan_amd.device import dptr, stream_handle
+    D, Ls, Us, b, off = _system(ni, nz, 'diagonal', ni + every)
+    for o, n in zip(off[:-1], nz):
+        gone = np.arange(0 if n % 2 else 1, n, 2)
+        for l in [*gone[::every]] if every else []:
+            D[o + l] = np.roll(D[o + l], 1 + l % (ni - 1), axis=0)
+        if every != 2 and n > 4:
+            D[o + 6 - n % 2] = np.roll(D[o + 6 - n % 2], 1, axis=0)
+    ref = np.concatenate([_dense(D[o:p], Ls[o:p], Us[o:p], b[o:p]) for o, p in zip(off[:-1], off[1:])])
+    d = [torch.as_tensor(a, device='cuda') for a in (D, Ls, Us, b)]
+    x = torch.empty_like(d[3])
+    info = torch.full((len(nz),), -1, dtype=torch.int32, device='cuda')
+    _lib.check(lib.vk_plan_set_factor_variant(plan.handle, 4), 'vk_plan_set_factor_variant')
+    for _ in range(2):                       # the second time over the first one's inverses and marks
+        x.zero_()
+        _lib.check(lib.vk_block_solve_system(plan.handle, cols.handle, *[dptr(t) for t in d], dptr(x), 0, dptr(info),
+                                             stream_handle()), 'vk_block_solve_system')
+        assert not info.cpu().numpy().any()
+        assert np.abs(x.cpu().numpy() - ref).max() < TOL * np.abs(ref).max()
+
+
+@gpu
+@pytest.mark.parametrize('ni', [112, 128])
+def test_cyclic_reduction_attempts_refused_blocks_once(ni):
+    """Blocks that refuse at their last pivots cost one level's attempt more than
+    blocks that refuse at their first (an attempt a level is a third more)."""
+    nz = [100]
+    torch, lib, plan, cols = _setup(ni, nz)
+    from vulcan_amd.device import dptr, stream_handle
+    rng = np.random.default_rng(ni)
+    kept = _blocks(ni, sum(nz), 1.0, rng)
+    late = kept.copy()
+    late[:, [ni - 2, ni - 1]] = late[:, [ni - 1, ni - 2]]
+    _lib.check(lib.vk_plan_set_factor_variant(plan.handle, 4), 'vk_plan_set_factor_variant')
+    zero = torch.zeros((sum(nz), ni), dtype=torch.float64, device='cuda')
+    D = [torch.as_tensor(np.ascontiguousarray(a), device='cuda') for a in (np.roll(kept, 1, axis=1), late)]
+    b, x = torch.ones_like(zero), torch.empty_like(zero)
+    best = [np.inf, np.inf]
+    for _ in range(8):
+        for q in (0, 1):
+            start, stop = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            for n in range(6):                # the first ones warm up the allocation
+                if n == 1:
+                    start.record()
+                _lib.check(lib.vk_block_solve_system(plan.handle, cols.handle, dptr(D[q]), dptr(zero), dptr(zero), dptr(b),
+                                                     dptr(x), 0, None, stream_handle()), 'vk_block_solve_system')
+            stop.record()
+            torch.cuda.synchronize()
+            best[q] = min(best[q], start.elapsed_time(stop) / 5)
+    print('refused at the first pivots %.3f ms, at the last %.3f ms' % tuple(best), flush=True)
+    assert best[1] < 1.17 * best[0]

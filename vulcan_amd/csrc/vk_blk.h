@@ -614,13 +614,6 @@ __device__ __forceinline__ void blk_load_schur(f64x4 (&acc)[BlkGrid<NB>::TBR][Bl
     if (Xn2) sub(cl2, Xn2, cn2);
 }
 
-// the workgroup's LDS for the inversions
-template <int NB>
-__device__ __forceinline__ BlkShared<NB> &blk_shared() {
-    __shared__ BlkShared<NB> sh;
-    return sh;
-}
-
 // How a kernel inverts the blocks that refuse diagonal pivots:
 enum BlkSearch {
     BLK_SEARCH_HERE,    // in place, with searched pivots (both inversions in the kernel's registers)
@@ -639,16 +632,19 @@ __device__ __forceinline__ bool blk_marked(const double *X) {
 }
 
 // X = the transposed inverse of D_l - diag(cl) Xn^T diag(cn) [- diag(cl2)
-// Xn2^T diag(cn2)]; false (uniform) where X is left marked
+// Xn2^T diag(cn2)], with search (uniform) without an attempt on the diagonal;
+// whether the diagonal's pivots were taken (uniform)
 template <int NB, int SEARCH>
 __device__ __forceinline__ bool blk_invert_schur(int ni, const double *__restrict__ Dl, const double *cl,
                                                  const double *Xn, const double *cn, const double *cl2,
                                                  const double *Xn2, const double *cn2, double *__restrict__ X,
-                                                 BlkShared<NB> &sh, int tag) {
+                                                 BlkShared<NB> &sh, int tag, bool search = false) {
     f64x4 acc[BlkGrid<NB>::TBR][BlkGrid<NB>::TBC];
     if constexpr (SEARCH != BLK_SEARCH_ONLY) {
-        blk_load_schur<NB>(acc, ni, Dl, cl, Xn, cn, cl2, Xn2, cn2);
-        if (blk_invert_diag<NB>(acc, ni, X, sh)) return true;
+        if (!search) {
+            blk_load_schur<NB>(acc, ni, Dl, cl, Xn, cn, cl2, Xn2, cn2);
+            if (blk_invert_diag<NB>(acc, ni, X, sh)) return true;
+        }
         if constexpr (SEARCH == BLK_SEARCH_MARK) {
             if (threadIdx.x == 0) blk_mark(X);
             return false;
@@ -656,7 +652,7 @@ __device__ __forceinline__ bool blk_invert_schur(int ni, const double *__restric
     }
     blk_load_schur<NB>(acc, ni, Dl, cl, Xn, cn, cl2, Xn2, cn2);
     blk_invert<NB>(acc, ni, X, sh, tag);
-    return true;
+    return false;
 }
 
 // acc = D_l - diag(cl) acc diag(cn) in the tile layout, acc holding the
