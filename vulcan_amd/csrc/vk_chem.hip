@@ -103,7 +103,8 @@ __device__ inline void log2d(double x, double &h, double &l) {
 }
 
 // c exp(t + lo) for |t| < 700, |lo| << 1: t = k ln 2 + r, the exponential's
-// series to r^13 / 13! (|r| < 0.35: 4e-18 left out)
+// series to r^13 / 13! (|r| < 0.35: 4e-18 left out).  The power of two comes
+// first: a factor below 2e-308 would round to its own coarse grid in the sum.
 __device__ inline double mul_exp(double c, double t, double lo) {
     const double k = rint(t * 1.4426950408889634);
     const double r = fma(-k, LN2_HI, t) + fma(-k, LN2_LO, lo);
@@ -119,13 +120,11 @@ __device__ inline double mul_exp(double c, double t, double lo) {
     q = fma(q, r, 1. / 24.);
     q = fma(q, r, 1. / 6.);
     q = fma(q, r, 0.5);
-    const double e = fma(q, r * r, r);
-    return ldexp(fma(c, e, c), (int)k);
+    const double e = fma(q, r * r, r), s = ldexp(c, (int)k);
+    return fma(s, e, s);
 }
 
 constexpr double EXP_FAST = 650.0;                    // |exponents| of the fast paths
-// both a factor and a result of mul_exp: it rounds the factor times 1 + e, on
-// the coarse grid below 2e-308, before the power of two
 __device__ inline bool rate_normal(double k) { return fabs(k) > 1e-280 && fabs(k) < 1e280; }
 
 // A T^n exp(-E/T)
@@ -133,7 +132,7 @@ __device__ inline double arrh(double A, double n, double E, const LayerRate &y) 
     const double q = E * y.rT, ql = fma(-q, y.T, E) * y.rT;              // E/T = q + ql
     const double h = n * y.lh, hl = fma(n, y.lh, -h) + n * y.ll;         // n log T = h + hl
     const double t = h - q, bb = t - h, tl = (h - (t - bb)) - (q + bb);  // h - q = t + tl
-    const bool in = rate_normal(A) && fabs(h) < EXP_FAST && fabs(q) < EXP_FAST && fabs(t) < EXP_FAST;   // false for NaN
+    const bool in = fabs(h) < EXP_FAST && fabs(q) < EXP_FAST && fabs(t) < EXP_FAST;   // false for NaN
     const double k = in ? mul_exp(A, t, tl + (hl - ql)) : 0.0;
     if (rate_normal(k)) return k;
     return A * pow(y.T, n) * exp(-E / y.T);
@@ -235,7 +234,7 @@ __global__ void __launch_bounds__(BLK, 4) k_rates(int L, int LG, int npairs, int
                 for (int q = 0; q < 4; q++) acc -= gl[a][sr[q]];
 #pragma unroll
                 for (int q = 0; q < 4; q++) acc += gl[a][sp[q]];
-                if (rate_normal(kf) && fabs(acc) < EXP_FAST && dn >= -1 && dn <= 1)
+                if (fabs(acc) < EXP_FAST && dn >= -1 && dn <= 1)
                     kr = mul_exp(kf, acc, 0.0) * (dn == 0 ? 1.0 : (dn == 1 ? y.rx : y.x));
                 if (!rate_normal(kr)) {
                     double K = exp(-acc);
