@@ -193,9 +193,11 @@ int vk_block_factor(const vk_plan *plan, const vk_columns *cols, const double *d
 /* Block-inversion kernel of the factorisation (no counterpart in the
  * reference, whose banded LU has one code path): VK_FACTOR_REGISTER keeps
  * the block in registers and runs one barrier-synchronised Gauss-Jordan
- * step per pivot; VK_FACTOR_BLOCKED groups the pivots in panels of 16,
- * factors each panel in one wave and applies the rank-16 Schur update on
- * FP64 MFMA (compiled for one or for two resident workgroups per CU);
+ * step per pivot; VK_FACTOR_BLOCKED takes the diagonal as pivots in panels of
+ * 8 or 16 that every wave factors for itself, or, where a block refuses them,
+ * searched pivots in panels of 16 factored by one wave, and applies the panel's
+ * Schur update on FP64 MFMA (compiled for one or for two resident workgroups
+ * per CU);
  * VK_FACTOR_WAVE holds the block in the registers of two waves and runs
  * one two-wave barrier per pivot step (small workgroups: several chains per
  * CU).  VK_FACTOR_BCR replaces the chain over layers by log2(nz) levels of
@@ -204,12 +206,12 @@ int vk_block_factor(const vk_plan *plan, const vk_columns *cols, const double *d
  * few columns; it keeps its own workspace, so it runs inside the
  * integrator and vk_block_solve_system, while vk_block_factor /
  * vk_block_solve reject it.  All give the solution to rounding; vk_tune_factor times every
- * variant on a synthetic system of the columns' shape (`reps` launches
- * each: one factorisation and two solves, milliseconds per repetition into
- * ms[VK_FACTOR_NVARIANTS], -1 for a variant that does not apply: the
- * two-wave kernel above ni = 112, cyclic reduction above 64 columns) and
- * keeps the
- * fastest in the plan. */
+ * variant on a synthetic system of the columns' shape whose blocks keep their
+ * diagonal as pivots, as an integration's do after its first steps (`reps`
+ * launches each: one factorisation and two solves, milliseconds per repetition
+ * into ms[VK_FACTOR_NVARIANTS], -1 for a variant that does not apply: the
+ * two-wave kernel above ni = 112, cyclic reduction above 64 columns) and keeps
+ * the fastest in the plan. */
 #define VK_FACTOR_REGISTER     0
 #define VK_FACTOR_BLOCKED      1   /* register budget for one workgroup per CU      */
 #define VK_FACTOR_BLOCKED_OCC2 2   /* register budget for two workgroups per CU     */

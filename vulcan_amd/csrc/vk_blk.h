@@ -21,7 +21,8 @@ struct BlkGrid {
 };
 
 // ---------------------------------------------------------------------------
-// Blocked Gauss-Jordan inversion on FP64 MFMA (factor variant 1)
+// Blocked Gauss-Jordan inversion on FP64 MFMA with searched pivots (factor
+// variants 1, 2 and 4, for blocks that refuse their diagonal as pivots, below)
 //
 // The pivot steps are grouped into panels of 16 columns.  One wave runs the
 // 16 pivot steps of a panel on the panel columns alone (rows spread over the
@@ -50,10 +51,19 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 // Pivots per panel of blk_invert_diag.  A pivot step broadcasts a row of the
 // panel and updates its columns, so narrow panels halve it, and twice as many
-// panels cost a round of publishing and two barriers each: measured 8 against
-// 16 with 48 species (80 columns' chains) 0.89 against 1.03 ms, 93 species one
-// block 38 against 31 us and 256 columns' chains 3.68 against 3.65 ms, 150
-// species one block 113 against 121 us and 80 columns' chains 7.4 against 7.6 ms.
+// panels cost a round of publishing and two barriers each.  Panels of 8 against
+// 16, chains of 1, 80 and 256 columns of 60 layers (us):
+//   30 species   182 : 192    194 : 208    266 : 322
+//   48           392 : 372    409 : 392    582 : 604
+//   49           459 : 444    481 : 461    768 : 674
+//   93           978 : 855   1051 : 930   1477 : 1445
+//   96          1037 : 911   1108 : 989   1484 : 1558
+//   97          1405 : 1519  1542 : 1621  2373 : 3145
+//   112         1615 : 1620  1759 : 1735  2585 : 3434
+//   128         1844 : 1868  1977 : 2003
+//   160         3143 : 3001  3373 : 3236
+// so 8 up to 48 and above 96 species, where up to 112 the registers it saves
+// also let two workgroups share a CU.
 template <int NB>
 constexpr int DIAG_PW = NB <= 3 || blk_nt(NB) > NT ? 8 : 16;
 

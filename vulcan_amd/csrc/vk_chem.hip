@@ -52,7 +52,7 @@ constexpr int RATE_LAYERS = 8;   // layers of a workgroup of k_rates, at most
 // each, of an argument held in two doubles, instead of a pow, an exp and a
 // division; arguments or results near the ends of the range (and NaN) take
 // the library functions.  256 columns (36 000 layers), 93 species, 620 pairs:
-// 493 us in two kernels, with g/RT written and read back, -> 255 us (bound by
+// 440 us in two kernels, with g/RT written and read back, -> 230 us (bound by
 // FP64 arithmetic; the 360 MB of rates take 75 us); the largest error against
 // 64 bits is the same 2.4e-15.
 
@@ -695,7 +695,9 @@ int vk_launch_rhs(const vk_plan *plan, const vk_columns *cols, const vk_atm *atm
                            plan->chem_ptr, plan->chem_ent, plan->ms, plan->alpha, a, y, k, atm->M, mode, mol, k1, dtc,
                            ysum, st, out);
     };
-    // two layers a workgroup where a CU holds eight such workgroups and still gets several
+    // two layers a workgroup where a CU holds eight such workgroups and still gets
+    // several (30 and 93 species: 3 008 layers, one each, 11.8 and 21.1 us, 3 072
+    // layers, two, 9.8 and 19.9)
     if (rhs_smem(plan, 2) <= 20 * 1024 && cols->L >= 12 * vk_device_cus())
         launch(k_rhs<2>, 2);
     else
